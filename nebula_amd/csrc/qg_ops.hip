@@ -4,6 +4,7 @@
 // kernels are written for CDNA4 wave64.
 #include "qg_internal.h"
 #include "qg_frag.h"
+#include "qg_exact.h"
 
 // The widths of the width-less entry points: a process-wide setting
 // (qg_moe_configure), which a thread may override for its own calls
@@ -107,26 +108,22 @@ __global__ __launch_bounds__(64) void mm_exact_kernel(float *__restrict__ out, c
     }
 }
 
-// qg_matmul for Q4_K and IQ4_NL rows with cols a multiple of 256, up to TT
-// tokens per block: the arithmetic of mm_exact_kernel (the same weight value
-// per element, lane j's chain over k = j (mod 32) in ascending k, the same
-// tree).  A block holds 8 RPL rows: 32-lane half h runs rows h, h + 8, ...
-// (RPL of them, sharing every x read).  Per chunk of KC columns: the rows'
-// weight bytes and the tile's x rows arrive by direct global->shared copies,
-// all in flight at once; then each group's d*s and -(dmin*m) (Q4_K) or each
-// block's d (IQ4_NL) is formed once into shared memory, and the rows' chains
-// run from shared memory.
+// qg_matmul for Q4_K and IQ4_NL rows with cols a multiple of 256 at up to 4
+// tokens: the arithmetic of mm_exact_kernel (the same weight value per
+// element, lane j's chain over k = j (mod 32) in ascending k, the same tree).
+// A block holds 8 rows, one per 32-lane half.  Per chunk of KC columns: the
+// rows' weight bytes and the tokens' x rows arrive by direct global->shared
+// copies, all in flight at once; then each group's d*s and -(dmin*m) (Q4_K) or
+// each block's d (IQ4_NL) is formed once into shared memory, and the rows'
+// chains run from shared memory.
 template <int TT> struct MmTile;
 template <> struct MmTile<1> { static constexpr int KC = 4096; };
 template <> struct MmTile<4> { static constexpr int KC = 2048; };
-template <> struct MmTile<8> { static constexpr int KC = 1024; };
-template <> struct MmTile<16> { static constexpr int KC = 512; };
-template <> struct MmTile<20> { static constexpr int KC = 512; };
 
-template <int TYPE, int TT, int RPL, int KCO = 0>
+template <int TYPE, int TT, int KCO = 0>
 __global__ __launch_bounds__(256) void mm_tile_kernel(float *__restrict__ out, const uint8_t *__restrict__ w, int rows,
                                                      int cols, const float *__restrict__ x, int nt, size_t stride) {
-    constexpr int KC = KCO ? KCO : MmTile<TT>::KC, RB = 8 * RPL;  // chunk columns; rows per block
+    constexpr int KC = KCO ? KCO : MmTile<TT>::KC, RB = 8;  // chunk columns; rows per block
     constexpr int WB = KC / 256 * 144;                                       // chunk bytes of a row
     constexpr int NS = TYPE == QT_Q4_K ? RB * (KC / 256) * 8 : RB * (KC / 32);  // scale entries per chunk
     __shared__ __attribute__((aligned(16))) float xs[TT * KC];    // [token][k], row stride kc
@@ -138,11 +135,9 @@ __global__ __launch_bounds__(256) void mm_tile_kernel(float *__restrict__ out, c
     const int r0 = blockIdx.x * RB;
     const int t0 = blockIdx.y * TT, n = min(nt - t0, TT);
     if (TYPE == QT_IQ4_NL && tid < 16) s_lut[tid] = (float)qg_iq4nl_lut[tid];
-    Acc<TT> a[RPL];
+    Acc<TT> a;
 #pragma unroll
-    for (int q = 0; q < RPL; q++)
-#pragma unroll
-        for (int t = 0; t < TT; t++) a[q].v[t] = 0.0f;
+    for (int t = 0; t < TT; t++) a.v[t] = 0.0f;
     for (int c0 = 0; c0 < cols; c0 += KC) {
         const int kc = min(KC, cols - c0), rb = kc / 256 * 144;  // this chunk's columns, bytes per row
         // the block's rows' bytes, contiguous per row (rows past the end repeat the last)
@@ -181,107 +176,115 @@ __global__ __launch_bounds__(256) void mm_tile_kernel(float *__restrict__ out, c
         __syncthreads();
         // tokens past the tile's n re-read its last row, rows past the end the
         // last row (their sums are not stored)
-        auto chains = [&](const float *wv, int k) {
+        auto chains = [&](float wv, int k) {
 #pragma unroll
-            for (int t = 0; t < TT; t++) {
-                const float xv = xs[min(t, n - 1) * kc + k];
-#pragma unroll
-                for (int q = 0; q < RPL; q++) a[q].v[t] = __builtin_fmaf(wv[q], xv, a[q].v[t]);
-            }
+            for (int t = 0; t < TT; t++) a.v[t] = __builtin_fmaf(wv, xs[min(t, n - 1) * kc + k], a.v[t]);
         };
         if (TYPE == QT_Q4_K) {
             const int nsb = kc / 256;
             for (int sb = 0; sb < nsb; sb++) {
 #pragma unroll
                 for (int gp = 0; gp < 4; gp++) {
-                    int byte[RPL];
-#pragma unroll
-                    for (int q = 0; q < RPL; q++) byte[q] = ws[(hw + 8 * q) * rb + sb * 144 + 16 + gp * 32 + j];
+                    const int byte = ws[hw * rb + sb * 144 + 16 + gp * 32 + j];
 #pragma unroll
                     for (int hi = 0; hi < 2; hi++) {
-                        float wv[RPL];
-#pragma unroll
-                        for (int q = 0; q < RPL; q++) {
-                            const float2 ds = s_sc[((hw + 8 * q) * nsb + sb) * 8 + 2 * gp + hi];
-                            wv[q] = __builtin_fmaf(ds.x, (float)((byte[q] >> (hi * 4)) & 15), ds.y);
-                        }
-                        chains(wv, sb * 256 + (2 * gp + hi) * 32 + j);
+                        const float2 ds = s_sc[(hw * nsb + sb) * 8 + 2 * gp + hi];
+                        chains(__builtin_fmaf(ds.x, (float)((byte >> (hi * 4)) & 15), ds.y), sb * 256 + (2 * gp + hi) * 32 + j);
                     }
                 }
             }
         } else {
             const int nb = kc / 32;
             for (int b = 0; b < nb; b++) {
-                float wv[RPL];
-#pragma unroll
-                for (int q = 0; q < RPL; q++) {
-                    const int r = hw + 8 * q;
-                    const int qq = (ws[r * rb + b * 18 + 2 + (j & 15)] >> ((j >> 4) * 4)) & 15;
-                    wv[q] = s_d[r * nb + b] * s_lut[qq];
-                }
-                chains(wv, b * 32 + j);
+                const int qq = (ws[hw * rb + b * 18 + 2 + (j & 15)] >> ((j >> 4) * 4)) & 15;
+                chains(s_d[hw * nb + b] * s_lut[qq], b * 32 + j);
             }
         }
         __syncthreads();  // the chunk's buffers are rewritten next
     }
+    const int row = r0 + hw;
 #pragma unroll
-    for (int q = 0; q < RPL; q++) {
-        const int row = r0 + hw + 8 * q;
-#pragma unroll
-        for (int t = 0; t < TT; t++) {
-            const float s = qg_tree32(a[q].v[t]);
-            if (j == 0 && t < n && row < rows) out[(size_t)(t0 + t) * rows + row] = s;
-        }
+    for (int t = 0; t < TT; t++) {
+        const float s = qg_tree32(a.v[t]);
+        if (j == 0 && t < n && row < rows) out[(size_t)(t0 + t) * rows + row] = s;
     }
 }
 
-// Two rows per lane halve the shared-memory reads per product (they pay off
-// for the long token tiles), when the matrix still fills 512 blocks.
 template <int TYPE, int TT>
 void launch_mm_tile(float *out, const uint8_t *w, int rows, int cols, const float *x, int nt, size_t stride, hipStream_t s) {
-    const int ty = (nt + TT - 1) / TT;
-    const dim3 g8((rows + 7) / 8, ty);
-    if constexpr (TT >= 16) {
-        if (((rows + 15) / 16) * ty >= 512) {
-            mm_tile_kernel<TYPE, TT, 2><<<dim3((rows + 15) / 16, ty), 256, 0, s>>>(out, w, rows, cols, x, nt, stride);
-            return;
-        }
-    } else if constexpr (TT == 1) {
+    const dim3 grid((rows + 7) / 8, (nt + TT - 1) / TT);
+    if constexpr (TT == 1) {
         if (cols <= 2560) {
             // one chunk of at most 2560 columns: a third less shared memory than
             // the 4096-column chunk, so 5 blocks per CU stay resident instead of 3
-            mm_tile_kernel<TYPE, 1, 1, 2560><<<g8, 256, 0, s>>>(out, w, rows, cols, x, nt, stride);
+            mm_tile_kernel<TYPE, 1, 2560><<<grid, 256, 0, s>>>(out, w, rows, cols, x, nt, stride);
             return;
         }
         if (cols > 4096 && cols <= 6144) {
             // one chunk instead of two (one copy round trip per block)
-            mm_tile_kernel<TYPE, 1, 1, 6144><<<g8, 256, 0, s>>>(out, w, rows, cols, x, nt, stride);
+            mm_tile_kernel<TYPE, 1, 6144><<<grid, 256, 0, s>>>(out, w, rows, cols, x, nt, stride);
             return;
         }
     } else {
         if (cols <= 2560) {
-            // two 1280-column chunks: 5 (4 tokens) or 3 (8 tokens) blocks per CU
-            // instead of 3 or 4, at the same or fewer copy rounds
-            mm_tile_kernel<TYPE, TT, 1, 1280><<<g8, 256, 0, s>>>(out, w, rows, cols, x, nt, stride);
+            // two 1280-column chunks: 5 blocks per CU instead of 3, at the same
+            // number of copy rounds
+            mm_tile_kernel<TYPE, TT, 1280><<<grid, 256, 0, s>>>(out, w, rows, cols, x, nt, stride);
             return;
         }
     }
-    mm_tile_kernel<TYPE, TT, 1><<<g8, 256, 0, s>>>(out, w, rows, cols, x, nt, stride);
+    mm_tile_kernel<TYPE, TT><<<grid, 256, 0, s>>>(out, w, rows, cols, x, nt, stride);
+}
+
+// qg_matmul on the fp32 matrix cores (qg_exact.h).  Tiles: 16 rows x 16 or 20
+// tokens (3 workgroups per CU), or 32 x 32 (2 per CU, half the operand reads
+// and decoding per product).  Estimated cost of a launch in units of one full
+// round of the small tile, fitted to 2560-column timings: 32 x 32 rounds of
+// 512 workgroups take twice as long (31 against 16 us), 1.4 times while every
+// CU has one (22 us); so the large tile is taken where it saves rounds (z 6144
+// x 2560, 300 tokens: 126 against 163 us) and the small one where the large
+// leaves CUs idle (out 2560 x 6144, 33 tokens: 34 against 55 us).
+template <int TYPE>
+void launch_xm(float *out, const uint8_t *w, int rows, int cols, const float *x, int nt, size_t stride, hipStream_t s) {
+    XmArgs A{out, rows, w, stride, rows, cols, x, nt, nullptr, 0, 0};
+    const int nrt = (rows + 15) / 16;
+    const long b16 = (long)nrt * ((nt + 15) / 16), b32 = (long)((rows + 31) / 32) * ((nt + 31) / 32);
+    if (nt > 20 && (b32 <= 256 ? 14 : 20 * ((b32 + 511) / 512)) <= 10 * ((b16 + 767) / 768)) {
+        if constexpr (TYPE != QT_Q8_0) {
+            xm_run<TYPE, 2, 0, 2, 1, 2, 4, 4>(A, s);
+            return;
+        }
+    }
+    constexpr int CH = TYPE == QT_F32 ? 1 : 2, XR = TYPE == QT_F32 ? 3 : 2;  // F32 rows may be an odd number of chunks
+    if (nt > 16 && nt <= 20) xm_run<TYPE, 1, 1, 1, CH, XR, 4, 4>(A, s);
+    else xm_run<TYPE, 1, 0, 1, CH, XR, 4, 4>(A, s);
 }
 
 template <int TYPE>
 void launch_mm_exact(float *out, const uint8_t *w, int type, int rows, int cols, const float *x, int nt, size_t stride,
                      const uint8_t *extra, hipStream_t s) {
+    // 16-byte copies need 16-byte aligned rows and x; the matrix-core tiles'
+    // row offsets are 32 bits wide
+    const bool aligned = !extra && (((uintptr_t)w | (uintptr_t)x | stride) & 15) == 0 && cols <= 1 << 20;
     if constexpr (TYPE == QT_Q4_K || TYPE == QT_IQ4_NL) {
-        // the tiled kernel's 16-byte copies need 16-byte aligned rows and x
-        if (!extra && cols % 256 == 0 && (((uintptr_t)w | (uintptr_t)x | stride) & 15) == 0) {
-        if (nt == 1) launch_mm_tile<TYPE, 1>(out, w, rows, cols, x, nt, stride, s);
-        else if (nt <= 4) launch_mm_tile<TYPE, 4>(out, w, rows, cols, x, nt, stride, s);
-        else if (nt <= 8) launch_mm_tile<TYPE, 8>(out, w, rows, cols, x, nt, stride, s);
-        else if (nt <= 16) launch_mm_tile<TYPE, 16>(out, w, rows, cols, x, nt, stride, s);
-        else launch_mm_tile<TYPE, 20>(out, w, rows, cols, x, nt, stride, s);
-        return;
+        if (aligned && cols % 256 == 0) {
+            // the vector chains up to 4 tokens (Q4_K 10240 x 2560: 15.2 us at 4
+            // tokens against 20.9), the matrix cores from 5 on (8 tokens: 26.3
+            // against 21.2 us, 17: 40.4 against 27.4, 1000: 1392 against 613)
+            if (nt == 1) launch_mm_tile<TYPE, 1>(out, w, rows, cols, x, nt, stride, s);
+            else if (nt <= 4) launch_mm_tile<TYPE, 4>(out, w, rows, cols, x, nt, stride, s);
+            else launch_xm<TYPE>(out, w, rows, cols, x, nt, stride, s);
+            return;
         }
+    }
+    if constexpr (TYPE == QT_Q8_0) {
+        // 10240 x 2560: 59 against 19 us at 1 token, 187 against 28 at 17
+        if (aligned && cols % 256 == 0) { launch_xm<TYPE>(out, w, rows, cols, x, nt, stride, s); return; }
+    }
+    if constexpr (TYPE == QT_F32) {
+        // 32 tokens and fewer: too few tiles of the router's 512 rows (512 x
+        // 2048: 17 tokens 5.3 against 9.3 us, 40 tokens 8.3 against 6.8)
+        if (aligned && cols % 128 == 0 && nt > 32) { launch_xm<TYPE>(out, w, rows, cols, x, nt, stride, s); return; }
     }
     dim3 grid((rows + 1) / 2, 1);
     if (nt == 1) { mm_exact_kernel<TYPE, 1><<<grid, 64, 0, s>>>(out, w, type, rows, cols, x, nt, stride, extra); return; }
@@ -493,6 +496,7 @@ int qg_launch_matmul_exact(float *out, const uint8_t *w, int type, int rows, int
     case QT_F32: launch_mm_exact<QT_F32>(out, w, type, rows, cols, x, nt, stride, extra, s); break;
     case QT_Q4_K: launch_mm_exact<QT_Q4_K>(out, w, type, rows, cols, x, nt, stride, extra, s); break;
     case QT_IQ4_NL: launch_mm_exact<QT_IQ4_NL>(out, w, type, rows, cols, x, nt, stride, extra, s); break;
+    case QT_Q8_0: launch_mm_exact<QT_Q8_0>(out, w, type, rows, cols, x, nt, stride, extra, s); break;
     default: launch_mm_exact<-1>(out, w, type, rows, cols, x, nt, stride, extra, s); break;
     }
     return hipGetLastError();
