@@ -236,21 +236,14 @@ void launch_mm_tile(float *out, const uint8_t *w, int rows, int cols, const floa
     mm_tile_kernel<TYPE, TT><<<grid, 256, 0, s>>>(out, w, rows, cols, x, nt, stride);
 }
 
-// qg_matmul on the fp32 matrix cores (qg_exact.h).  Tiles: 16 rows x 16 or 20
-// tokens (3 workgroups per CU), or 32 x 32 (2 per CU, half the operand reads
-// and decoding per product).  Estimated cost of a launch in units of one full
-// round of the small tile, fitted to 2560-column timings: 32 x 32 rounds of
-// 512 workgroups take twice as long (31 against 16 us), 1.4 times while every
-// CU has one (22 us); so the large tile is taken where it saves rounds (z 6144
-// x 2560, 300 tokens: 126 against 163 us) and the small one where the large
-// leaves CUs idle (out 2560 x 6144, 33 tokens: 34 against 55 us).
+// qg_matmul on the fp32 matrix cores (qg_exact.h): the wide tile where it is
+// the faster, else 16 rows x 16 tokens, with 4 more tokens in the same tile at
+// 17..20 (2560 x 6144, 17 tokens: 27 us against 34 in two tiles).
 template <int TYPE>
 void launch_xm(float *out, const uint8_t *w, int rows, int cols, const float *x, int nt, size_t stride, hipStream_t s) {
-    XmArgs A{out, rows, w, stride, rows, cols, x, nt, nullptr, 0, 0};
-    const int nrt = (rows + 15) / 16;
-    const long b16 = (long)nrt * ((nt + 15) / 16), b32 = (long)((rows + 31) / 32) * ((nt + 31) / 32);
-    if (nt > 20 && (b32 <= 256 ? 14 : 20 * ((b32 + 511) / 512)) <= 10 * ((b16 + 767) / 768)) {
-        if constexpr (TYPE != QT_Q8_0) {
+    const XmArgs A{out, rows, w, stride, rows, cols, x, nt, nullptr, 0, 0};
+    if constexpr (TYPE != QT_Q8_0) {
+        if (nt > 20 && xm_wide(rows, nt)) {
             xm_run<TYPE, 2, 0, 2, 1, 2, 4, 4>(A, s);
             return;
         }

@@ -6,11 +6,11 @@
 // per-expert row lists built on the device.
 //
 // Kernels per layer:
-//   P1 router   : exact-order router GEMM (the summation order of
-//                 cpu.c:122-139, so logits and routing are bit-exact), rows
-//                 0..511 plus the shared gate vector, + optional bias.
-//   P2 route    : a wave per token: top-10, coverage/prune, flags, and the
-//                 token's fp16 activation planes.
+//   P1 router   : exact-order router GEMM on the fp32 matrix cores (the
+//                 summation order of cpu.c:122-139, so logits and routing are
+//                 bit-exact), + optional bias.
+//   P2 route    : two waves per token: top-10, coverage/prune, flags, and the
+//                 token's fp16 activation planes and shared-gate logit.
 //   P2b count   : per 32-token chunk, the per-expert token masks, whose
 //                 popcounts are the chunk's histogram counts[chunk][e].
 //   P3 scan     : per-expert totals, CSR offsets, per-chunk bases (exclusive
@@ -44,6 +44,7 @@
 // hit 16 different bank groups.
 #include "qg_internal.h"
 #include "qg_frag.h"
+#include "qg_exact.h"
 #include <hip/hip_ext.h>
 #include <type_traits>
 
@@ -129,99 +130,20 @@ __global__ __launch_bounds__(256) void pf_norm_kernel(float *xn, const float *x,
 }
 
 // ---------------- P1: router logits ----------------
-// logits[t][r] = sum_k R[r][k] x[t][k] in the order of cpu.c:122-139: chain j
-// (0..31) accumulates k = j, j+32, ... ascending with fused multiply-add,
-// then the tree 16/8/4/2/1 of gpu.cu:154-180 (qg_tree32).  Block = 16 waves
-// = 64 tokens x 32 rows; half-wave h of wave w owns 8 tokens (w % 8) x 8 rows
-// ((w / 8) * 2 + h), lane j of the half-wave owns chain j of all 64 of its
-// outputs (112 registers: four waves per SIMD hide the shared-memory reads).
-// K chunks of 128 columns of both operands are staged in shared memory
-// (direct global->shared copies, double-buffered); the two half-waves of a
-// wave read the same token rows (broadcast) and different router rows.  The
-// final tree runs as an exchange butterfly: at offset s the lanes with bit s
-// clear keep the lower half of their outputs, the others the upper half, and
-// each adds its partner's value; float addition is commutative, so every
-// output is the same sum, paired the same way, as lane 0's of qg_tree32.
-// Lane j ends with outputs 2j, 2j+1 = token j/4, rows 2(j&3), 2(j&3)+1.
-constexpr int RT_TOK = 64, RT_ROWS = 32, RT_KC = 128;
-constexpr int RT_TT = 8;                          // tokens per half-wave (x 8 rows: RT_TT * 8 chains per lane)
-constexpr int RT_WAVES = (RT_TOK / RT_TT) * (RT_ROWS / 8) / 2;
-constexpr int RT_LDS = 2 * (RT_ROWS + RT_TOK) * RT_KC * 4;
-
-struct RouterArgs {
-    const float *x; int nt, D, rows;
-    const float *router, *sh_row;    // rows 0..511, row 512 (the shared gate vector) when rows == 513
-    const float *bias;               // added to rows 0..511, or null
-    float *logits;                   // [nt][rows]
-};
-
-__global__ __launch_bounds__(64 * RT_WAVES) void pf_router_kernel(RouterArgs A) {
-    constexpr int NTG = RT_TOK / RT_TT, V = RT_TT / 4;  // token groups; outputs per lane after the tree
-    extern __shared__ uint4 s_dyn[];
-    float *sw = (float *)s_dyn;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, h = lane >> 5, j = lane & 31;
-    const int tg = wave % NTG, rg = (wave / NTG) * 2 + h;
-    const int t0 = blockIdx.x * RT_TOK, r0 = blockIdx.y * RT_ROWS, nch = A.D / RT_KC;
-    auto stage = [&](int c, int b) {
-        // 32 router rows then 64 token rows, 512 B each: 48 copies of two rows
-        for (int q = wave; q < (RT_ROWS + RT_TOK) / 2; q += RT_WAVES) {
-            const int R = 2 * q + h;
-            const float *src;
-            if (R < RT_ROWS) {
-                const int r = min(r0 + R, A.rows - 1);
-                src = r == QG_EXPERTS ? A.sh_row : A.router + (size_t)r * A.D;
-            } else {
-                src = A.x + (size_t)min(t0 + R - RT_ROWS, A.nt - 1) * A.D;
-            }
-            dma16(src + (size_t)c * RT_KC + 4 * j, sw + (size_t)b * (RT_ROWS + RT_TOK) * RT_KC + q * 2 * RT_KC);
-        }
-    };
-    float acc[RT_TT][8];
-#pragma unroll
-    for (int t = 0; t < RT_TT; t++)
-#pragma unroll
-        for (int r = 0; r < 8; r++) acc[t][r] = 0.0f;
-    stage(0, 0);
-    for (int c = 0; c < nch; c++) {
-        wait_vmem();
-        __syncthreads();
-        if (c + 1 < nch) stage(c + 1, (c + 1) & 1);
-        const float *W = sw + (size_t)(c & 1) * (RT_ROWS + RT_TOK) * RT_KC + rg * 8 * RT_KC;
-        const float *X = sw + (size_t)(c & 1) * (RT_ROWS + RT_TOK) * RT_KC + (RT_ROWS + tg * RT_TT) * RT_KC;
-#pragma unroll
-        for (int i = 0; i < RT_KC / 32; i++) {
-            float wv[8], xv[RT_TT];
-#pragma unroll
-            for (int r = 0; r < 8; r++) wv[r] = W[r * RT_KC + 32 * i + j];
-#pragma unroll
-            for (int t = 0; t < RT_TT; t++) xv[t] = X[t * RT_KC + 32 * i + j];
-#pragma unroll
-            for (int t = 0; t < RT_TT; t++)
-#pragma unroll
-                for (int r = 0; r < 8; r++) acc[t][r] = __builtin_fmaf(wv[r], xv[t], acc[t][r]);
-        }
-    }
-    // exchange butterfly over the 32 lanes of the half-wave; v[o], o = 8t + r
-    float *v = &acc[0][0];
-#pragma unroll
-    for (int s = 16, n = 8 * RT_TT; s >= 1; s >>= 1, n >>= 1) {
-        const bool up = (j & s) != 0;
-#pragma unroll
-        for (int q = 0; q < n / 2; q++) {
-            const float send = up ? v[q] : v[q + n / 2];
-            const float recv = __shfl_xor(send, s, 32);
-            v[q] = (up ? v[q + n / 2] : v[q]) + recv;
-        }
-    }
-    // lane j holds outputs o = V j .. V j + V - 1
-    const int t = t0 + tg * RT_TT + (V * j) / 8;
-    if (t < A.nt) {
-#pragma unroll
-        for (int q = 0; q < V; q++) {
-            const int r = r0 + rg * 8 + (V * j) % 8 + q;
-            if (r < A.rows) A.logits[(size_t)t * A.rows + r] = A.bias && r < QG_EXPERTS ? v[q] + A.bias[r] : v[q];
-        }
-    }
+// logits[t][r] = sum_k R[r][k] x[t][k] (+ bias[r]) for the 512 experts in the
+// order of cpu.c:122-139 on the fp32 matrix cores (qg_exact.h).  Tiles by
+// batch: 16 x 16 until the 32 x 32 ones fill the CUs (xm_wide), 64 tokens x 32
+// rows from 4096 tokens on, where a quarter fewer operand bytes per product
+// outweigh the single workgroup per CU (8192 tokens at D = 2048: 200 -> 176
+// us; 2048: no difference).  The scalar chains that this replaces were bound
+// by their shared-memory reads and filled 17 CUs per 64 tokens: 33 -> 7 us at
+// 40 tokens, 89 -> 49 at 2048.
+template <int N16, int RR, int XR, int OCC>
+void pf_router(XmArgs A, hipStream_t s) {
+    using S = XmShape<QT_F32, N16, 0, RR, 1, XR, 1>;
+    A.ntt = (A.nt + S::TOK - 1) / S::TOK;
+    A.nrt = QG_EXPERTS / S::ROWS;
+    pf_launch(0, xm_kernel<QT_F32, N16, 0, RR, 1, XR, 1, OCC>, dim3(A.ntt * A.nrt), dim3(512), S::LDS, s, A);
 }
 
 // ---------------- P2: routing and activation planes ----------------
@@ -230,6 +152,7 @@ struct RouteArgs {
     const uint8_t *resident; double thr;
     int *ids; float *w; uint8_t *flags_out; int *flag; int *missing; double *mass;
     const float *x; int D; _Float16 *xp, *xsp;
+    const float *sh_row; float *sh_logit;   // shared gate vector and its logits (sh_logit[t * ld]), or null
     int8_t *xi8; float *xsc;          // int8 planes and row scales (the int8 dense pass), or null
 };
 
@@ -260,7 +183,8 @@ QG_DEV void token_planes_i8(const float *xr, int D, int lane, int8_t *hi, int8_t
 
 // Two waves per token (block = 4 tokens): wave w < 4 routes token 4b + w
 // (top-10 of the (biased) logits, coverage/prune, flags) while wave w + 4
-// writes its fp16 hi/lo planes and 32-group sum planes.
+// writes its fp16 hi/lo planes and 32-group sum planes and the shared gate's
+// logit (lane j of a half-wave runs chain j, in the router's order).
 __global__ __launch_bounds__(512) void pf_route_kernel(RouteArgs A) {
     __shared__ __align__(16) float s_rv[4][QG_ROUTE_SCRATCH];
     __shared__ __align__(16) int s_ri[4][QG_ROUTE_SCRATCH];
@@ -269,6 +193,14 @@ __global__ __launch_bounds__(512) void pf_route_kernel(RouteArgs A) {
     if (wave >= 4) {  // the token's activation planes, beside its routing
         _Float16 *hi = A.xp + (size_t)t * 2 * A.D, *shi = A.xsp + (size_t)t * 2 * (A.D / 32);
         token_planes(A.x + (size_t)t * A.D, A.D, false, 1.0f, lane, hi, hi + A.D, shi, shi + A.D / 32, nullptr);
+        if (A.sh_row) {
+            const float *xr = A.x + (size_t)t * A.D + (lane & 31), *gr = A.sh_row + (lane & 31);
+            float a = 0.0f;
+#pragma unroll 16
+            for (int k = 0; k < A.D; k += 32) a = __builtin_fmaf(gr[k], xr[k], a);
+            a = qg_tree32(a);
+            if (lane == 0) A.sh_logit[(size_t)t * A.ld] = a;
+        }
         if (A.xi8) token_planes_i8(A.x + (size_t)t * A.D, A.D, lane, A.xi8 + (size_t)t * 2 * A.D, A.xi8 + (size_t)t * 2 * A.D + A.D, A.xsc + t);
         return;
     }
@@ -1611,16 +1543,19 @@ int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsig
         if ((rc = hipGetLastError())) return rc;
         x = xn;
     }
-    // P1: router logits in the reference's order (+ shared gate row, + bias)
-    RouterArgs R{x, nt, D, rows, L->router, sh ? L->sh_gate_inp : nullptr, L->router_bias, logits};
-    pf_launch(0, pf_router_kernel, dim3((nt + RT_TOK - 1) / RT_TOK, (rows + RT_ROWS - 1) / RT_ROWS), dim3(64 * RT_WAVES), RT_LDS, s, R);
+    // P1: router logits in the reference's order (+ bias)
+    const XmArgs R{logits, rows, (const uint8_t *)L->router, (size_t)D * 4, QG_EXPERTS, D, x, nt, L->router_bias, 0, 0};
+    if (nt >= 4096) pf_router<4, 2, 2, 2>(R, s);
+    else if (xm_wide(QG_EXPERTS, nt)) pf_router<2, 2, 2, 4>(R, s);
+    else pf_router<1, 1, 3, 4>(R, s);
     if ((rc = hipGetLastError())) return rc;
     const int split = tl_pf_split;
     const bool i8 = split == 1;
     int8_t *xi8 = i8 ? (int8_t *)(ws + lay.xi8) : nullptr;
     float *xsc = i8 ? (float *)(ws + lay.xsc) : nullptr, *row_sx = i8 ? (float *)(ws + lay.row_sx) : nullptr;
     RouteArgs RA{nt, logits, rows, L->resident, L->threshold, ids, weights, flags, flag,
-                 (int *)(ws + lay.missing), (double *)(ws + lay.mass), x, D, xp, xsp, xi8, xsc};
+                 (int *)(ws + lay.missing), (double *)(ws + lay.mass), x, D, xp, xsp,
+                 sh ? L->sh_gate_inp : nullptr, logits + QG_EXPERTS, xi8, xsc};
     pf_launch(1, pf_route_kernel, dim3((nt + 3) / 4), dim3(512), 0, s, RA);
     if ((rc = hipGetLastError())) return rc;
     pf_launch(10, pf_count_kernel, dim3(nch), dim3(512), 0, s, counts, (int *)nullptr, (const int *)ids, (const int *)flag, nt);

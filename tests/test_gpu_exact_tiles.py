@@ -69,3 +69,18 @@ def test_exact_special_values(qgl, typ, nt):
     nan = np.isnan(want)
     np.testing.assert_array_equal(np.isnan(got), nan)
     np.testing.assert_array_equal(got[~nan].view('u4'), want[~nan].view('u4'))
+
+
+@pytest.mark.parametrize("nt", [18, 500, 4101])
+def test_prefill_router_tiles(qgl, nt):
+    """The prefill router's three tile choices, each with a ragged last tile:
+    ids and weights of every token bit for bit, and the outputs (with the
+    shared expert, whose gate logit the routing kernel forms) on sampled rows."""
+    import test_gpu_prefill as P
+    from nebula_amd import synth
+    spec = synth.LayerSpec(seed=470, width=512, ff=128, gate_type=12, up_type=12, down_type=20, shared=True, sh_types=(12, 12, 20))
+    L, H = synth.build_layer(spec), P.host_layer(spec)
+    x = synth.inputs(480 + nt, nt, 512)
+    fw = P.forward(L, x)
+    P.check_routing(fw, H, x)
+    P.check_outputs(fw, L, H, x, P.sample_rows(nt, 10, nt), f"512/128 B={nt}")
