@@ -709,46 +709,6 @@ constexpr int GU3_MAXX = MAX_TILES + 1;                           // experts in 
 static_assert((size_t)(5 * GU3_MAXX + 1 + MS) * 4 <= GU3_RED_BYTES, "the expert list and ids fit a partial-sum buffer");
 constexpr int GU3_COST = 1;                                       // a block's copy cost in units of one tile's compute (measured best of 0..8)
 
-// The block's products for the M tiles: y[cb][m] = the wave's partial sums
-// over its superblock for the 16 gate (cb 0) or up (cb 1) rows, column j,
-// as (token 2kq, token 2kq + 1) with the hi and lo plane rows added.
-template <int M>
-QG_DEV void gu3_products(const uint4 *wb, const qg_half8 (&af)[GU3_MAXT][8], const qg_half8 (&sf)[GU3_MAXT], int j,
-                         int kq, float2 (&y)[2][GU3_MAXT]) {
-#pragma unroll
-    for (int cb = 0; cb < 2; cb++) {
-        const int row = cb * 16 + j, rot = row >> 3;
-        // piece c of the row (0: header, 1..8: nibbles), rotated by row / 8
-        auto piece = [&](int c) { const int x = c + rot; return wb[9 * row + (x >= 9 ? x - 9 : x)]; };
-        const Q4kHeader h = q4k_header(piece(0));
-        const uint4 ch0 = piece(1 + kq), ch1 = piece(5 + kq);
-        qg_half2 scA, ofA, scB, ofB;  // scales of groups gA, gA + 1 and gB, gB + 1
-        gq_scales(h.S[0], kq, scA, ofA);
-        gq_scales(h.S[1], kq, scB, ofB);
-        qg_f4 p0[M], p1[M], mm[M];
-#pragma unroll
-        for (int m = 0; m < M; m++) p0[m] = p1[m] = mm[m] = qg_f4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int f = 0; f < 4; f++) {
-            const qg_half8 b0 = gq_frag(ch0, f, scA[f >> 1], ofA[f >> 1]), b1 = gq_frag(ch1, f, scB[f >> 1], ofB[f >> 1]);
-#pragma unroll
-            for (int m = 0; m < M; m++) {
-                p0[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[m][f], b0, p0[m], 0, 0, 0);
-                p1[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[m][4 + f], b1, p1[m], 0, 0, 0);
-            }
-        }
-        const qg_half8 bm = q4k_min_frag(h);
-#pragma unroll
-        for (int m = 0; m < M; m++) {
-            mm[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sf[m], bm, mm[m], 0, 0, 0);
-            float v[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) v[i] = __builtin_fmaf(h.d, p0[m][i] + p1[m][i], -h.dmin * mm[m][i]);
-            y[cb][m] = make_float2(v[0] + v[1], v[2] + v[3]);
-        }
-    }
-}
-
 // This wave's copies of F block rb of an expert (gate rows gm, up rows um)
 // into its ring slot: each row's 144 bytes of the wave's superblock as one
 // run, rotated by row / 8 pieces so that the 16 rows of a fragment read
@@ -835,7 +795,7 @@ QG_DEV void gu3_run(const GuArgs &A, const int *ids, int e, int rb0, int rb1, co
         else if (ahead == 1) wait_vmem_but<GU3_CPB>();
         else wait_vmem();
         float2 y[2][GU3_MAXT];
-        gu3_products<M>(ring + (size_t)(it % GU3_RING) * GU3_SLOT, af, sf, j, kq, y);
+        ksplit_products<M>(ring + (size_t)(it % GU3_RING) * GU3_SLOT, af, sf, j, kq, y);
         // partial sums alternate between two buffers: block it + 2 rewrites
         // this one only after every wave has passed block it + 1's barrier,
         // so this block's epilogue needs no barrier of its own

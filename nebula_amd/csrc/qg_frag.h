@@ -94,6 +94,49 @@ QG_DEV qg_half8 gq_frag(uint4 c, int f, _Float16 sc, _Float16 of) {
     return r;
 }
 QG_DEV qg_half8 ld_frag(const _Float16 *p) { return __builtin_bit_cast(qg_half8, *(const uint4 *)p); }
+// A wave's products of one superblock of 16 gate and 16 up Q4_K rows (9 pieces
+// of 16 bytes each at wb, rotated by row / 8) with M tiles of 8 token rows
+// (af: their hi and lo planes as the 16 rows of a fragment, sf: the planes of
+// the group sums): y[cb][m] = the partial sums for the 16 gate (cb 0) or up (cb 1) rows, column j,
+// as (token 2kq, token 2kq + 1) with the hi and lo plane rows added.
+template <int M, int MT>
+QG_DEV void ksplit_products(const uint4 *wb, const qg_half8 (&af)[MT][8], const qg_half8 (&sf)[MT], int j, int kq,
+                            float2 (&y)[2][MT]) {
+    static_assert(M <= MT, "tiles");
+#pragma unroll
+    for (int cb = 0; cb < 2; cb++) {
+        const int row = cb * 16 + j, rot = row >> 3;
+        // piece c of the row (0: header, 1..8: nibbles), rotated by row / 8
+        auto piece = [&](int c) { const int x = c + rot; return wb[9 * row + (x >= 9 ? x - 9 : x)]; };
+        const Q4kHeader h = q4k_header(piece(0));
+        const uint4 ch0 = piece(1 + kq), ch1 = piece(5 + kq);
+        qg_half2 scA, ofA, scB, ofB;  // scales of groups gA, gA + 1 and gB, gB + 1
+        gq_scales(h.S[0], kq, scA, ofA);
+        gq_scales(h.S[1], kq, scB, ofB);
+        qg_f4 p0[M], p1[M], mm[M];
+#pragma unroll
+        for (int m = 0; m < M; m++) p0[m] = p1[m] = mm[m] = qg_f4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int f = 0; f < 4; f++) {
+            const qg_half8 b0 = gq_frag(ch0, f, scA[f >> 1], ofA[f >> 1]), b1 = gq_frag(ch1, f, scB[f >> 1], ofB[f >> 1]);
+#pragma unroll
+            for (int m = 0; m < M; m++) {
+                p0[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[m][f], b0, p0[m], 0, 0, 0);
+                p1[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[m][4 + f], b1, p1[m], 0, 0, 0);
+            }
+        }
+        const qg_half8 bm = q4k_min_frag(h);
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+            mm[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sf[m], bm, mm[m], 0, 0, 0);
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) v[i] = __builtin_fmaf(h.d, p0[m][i] + p1[m][i], -h.dmin * mm[m][i]);
+            y[cb][m] = make_float2(v[0] + v[1], v[2] + v[3]);
+        }
+    }
+}
+
 // Raw buffer loads (no stride; the byte range is the descriptor's record
 // count): an offset past the range reads zeros with no memory access.
 // QG_BUF_DW3: descriptor word 3 for gfx9 raw buffers (32-bit data format).

@@ -26,6 +26,8 @@
 //   P6 down     : persistent grouped GEMM, one launch (three when the shared
 //                 expert's down format differs); item = (group, 64-row tile,
 //                 256 D rows); y rows written to the selection's slot.
+//                 Smaller batches, whose experts have few rows, take the
+//                 kernels of qg_sparse.h for P5 and P6.
 //   P7 combine  : out[t] = sum over ranks k of w[t,k]*y[t,k] in rank order,
 //                 + sigmoid-gated shared expert, + optional residual.
 // Groups are the 512 experts plus the shared expert (group 512, every token).
@@ -45,6 +47,7 @@
 #include "qg_internal.h"
 #include "qg_frag.h"
 #include "qg_exact.h"
+#include "qg_sparse.h"
 #include <hip/hip_ext.h>
 #include <type_traits>
 
@@ -1407,6 +1410,43 @@ __global__ __launch_bounds__(512, 1) void pf_gateup_kernel(GuArgs A) {
     }
 }
 
+// The kernels of qg_sparse.h for batches whose experts have few rows, where
+// they stream and convert the weights in fewer instructions; above, the 64-row
+// tiles of pf_gateup_kernel and the down kernels re-read no weights.  The batch
+// limits lie where the two cross (uniform routing, us, 64-row tiles / these):
+//   gate/up D 2048: 40 tokens 111 / 67, 400 194 / 144, 1000 245 / 204, 1500 284 / 300
+//           D 2560: 60 tokens 200 / 147, 301 283 / 221, 600 297 / 271, 1200 366 / 471
+//           D 1024: 100 tokens 54 / 37, 600 66 / 53, 1500 80 / 97
+//   down Q4_K   F 512: 40 tokens 73 / 39, 600 136 / 93, 1500 189 / 170, 2500 249 / 260
+//        IQ4_NL F 512: 40 tokens 71 / 48, 400 129 / 116, 800 145 / 193
+//        IQ4_NL F 640: 60 tokens 131 / 89, 301 185 / 143, 600 197 / 233
+//        F 256, Q4_K: 1500 tokens 60 / 64; IQ4_NL: 100 tokens 35 / 28, 600 45 / 41, 1500 59 / 76
+// Runs of two tiles hold the mid fragments of K = 512 in registers for Q4_K; the
+// IQ4_NL conversion needs the registers, so it takes one tile there (with two,
+// spills in the loop made 400 tokens 262 us).
+bool pf_gateup_sp(const SpGuArgs &A, int cus, hipStream_t s) {
+    if (A.D == 2048 && A.nt <= 1280) pf_launch(5, pf_gateup_sp_kernel<8, 3>, dim3(cus), dim3(512), SpGu<8, 3>::LDS, s, A);
+    else if (A.D == 2560 && A.nt <= 640) pf_launch(5, pf_gateup_sp_kernel<10, 2>, dim3(cus), dim3(640), SpGu<10, 2>::LDS, s, A);
+    else if (A.D == 1024 && A.nt <= 896) pf_launch(5, pf_gateup_sp_kernel<4, 2>, dim3(2 * cus), dim3(256), SpGu<4, 2>::LDS, s, A);
+    else return false;
+    return true;
+}
+bool pf_down_sp(const SpDnArgs &A, int fmt, int F, int cus, hipStream_t s) {
+    auto go = [&](auto FC, auto NC, int most) {
+        constexpr int FMT = decltype(FC)::value, NB = decltype(NC)::value, TM = FMT == QT_IQ4_NL && NB >= 16 ? 1 : 2;
+        if (A.nt > most) return false;
+        pf_launch(7, pf_down_sp_kernel<FMT, NB, TM>, dim3(cus), dim3(512), SpDn<FMT, NB>::LDS, s, A);
+        return true;
+    };
+    using Q4 = std::integral_constant<int, QT_Q4_K>;
+    using IQ = std::integral_constant<int, QT_IQ4_NL>;
+    using N8 = std::integral_constant<int, 8>;
+    using N16 = std::integral_constant<int, 16>;
+    using N20 = std::integral_constant<int, 20>;
+    if (fmt == QT_Q4_K) return F == 256 ? go(Q4{}, N8{}, 1280) : F == 512 ? go(Q4{}, N16{}, 2048) : false;
+    return F == 256 ? go(IQ{}, N8{}, 640) : F == 512 ? go(IQ{}, N16{}, 448) : F == 640 ? go(IQ{}, N20{}, 400) : false;
+}
+
 // ---------------- P7: combine ----------------
 struct CombArgs {
     int nt, D;
@@ -1577,7 +1617,12 @@ int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsig
         else pf_launch(slot, pf_gateup_kernel<false>, dim3(grid), dim3(512), PF_GQ_LDS, s, G);
         return hipGetLastError();
     };
-    if (split) {
+    const SpGuArgs GS{nt, D, F, offsets, row_token, (const uint8_t *)L->gate, (const uint8_t *)L->up,
+                      sh ? (const uint8_t *)L->sh_gate : nullptr, sh ? (const uint8_t *)L->sh_up : nullptr, qg_row_bytes_host(QT_Q4_K, D),
+                      xp, xsp, midp, msp, L->down_type, sh ? L->sh_down_type : L->down_type};
+    if (!split && pf_gateup_sp(GS, grid, s)) {
+        if ((rc = hipGetLastError())) return rc;
+    } else if (split) {
         if ((rc = gate_up(0, 1, i8, 4))) return rc;
         if ((rc = gate_up(1, 3, false, 5))) return rc;
     } else if ((rc = gate_up(0, 3, false, 5))) {
@@ -1590,7 +1635,11 @@ int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsig
         else pf_launch(slot, pf_down_iq_kernel, dim3(grid), dim3(512), PF_IQ_LDS, s, DA);
         return hipGetLastError();
     };
-    if (!sh || L->sh_down_type == L->down_type) {
+    const bool one_fmt = !sh || L->sh_down_type == L->down_type;
+    const SpDnArgs DS{nt, D, offsets, row_slot, (const uint8_t *)L->down, sh ? (const uint8_t *)L->sh_down : nullptr, midp, msp, slots};
+    if (one_fmt && pf_down_sp(DS, L->down_type, F, grid, s)) {
+        if ((rc = hipGetLastError())) return rc;
+    } else if (one_fmt) {
         if ((rc = down(0, 3, L->down_type, 7))) return rc;
     } else {  // the shared expert's down in its own format
         if ((rc = down(0, 1, L->down_type, 6))) return rc;

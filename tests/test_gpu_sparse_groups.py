@@ -1,0 +1,91 @@
+"""The prefill's kernels for short row lists (qg_sparse.h) where they can go
+wrong: groups of 1 row, of exactly and just over one tile and one run, few long
+groups among empty experts, with and without the shared expert, each width and
+down format; and the batch limits, where both kernels see the same rows.
+Outputs against the oracle at the layer's tolerance, routing bit for bit."""
+import sys
+
+import numpy as np
+import pytest
+
+import test_gpu_prefill as P
+from nebula_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+LAYERS = {
+    "1024-iq4": dict(seed=501, width=1024, ff=256, down_type=20, shared=True, sh_types=(12, 12, 20)),
+    "1024-q4k": dict(seed=502, width=1024, ff=256, down_type=12, shared=False),
+    "2048-iq4": dict(seed=503, width=2048, ff=512, down_type=20, shared=True, sh_types=(12, 12, 20)),
+    "2048-q4k": dict(seed=504, width=2048, ff=512, down_type=12, shared=True, sh_types=(12, 12, 12)),
+    "2560-iq4": dict(seed=505, width=2560, ff=640, down_type=20, shared=True, sh_types=(12, 12, 20)),
+}
+
+
+@pytest.fixture(scope="module", params=sorted(LAYERS))
+def layer(request, qgl):
+    spec = synth.LayerSpec(**LAYERS[request.param])
+    return synth.build_layer(spec), P.host_layer(spec)
+
+
+def one_context(seed, nt, width):
+    """Rows so alike that nearly every token selects the same experts: about
+    ten groups of nt rows."""
+    rng = np.random.default_rng(seed)
+    return synth.rmsnorm(rng.standard_normal(width)[None, :] + 0.01 * rng.standard_normal((nt, width)))
+
+
+@pytest.mark.parametrize("nt", [18, 24, 25, 33, 200])
+def test_sparse_long_groups(layer, nt):
+    L, H = layer
+    x = one_context(510 + nt, nt, L.spec.width)
+    fw = P.forward(L, x)
+    P.check_routing(fw, H, x)
+    P.check_outputs(fw, L, H, x, np.unique(np.r_[0, 7, 8, 15, 16, 17, nt - 1]), f"long groups D={L.spec.width} nt={nt}")
+
+
+@pytest.mark.parametrize("nt", [18, 61])
+def test_sparse_short_groups(layer, nt):
+    L, H = layer
+    x = synth.inputs(520 + nt, nt, L.spec.width)
+    fw = P.forward(L, x)
+    P.check_routing(fw, H, x)
+    P.check_outputs(fw, L, H, x, P.sample_rows(nt, 8, nt), f"short groups D={L.spec.width} nt={nt}")
+
+
+@pytest.mark.parametrize("limit", [400, 448, 640, 896, 1280, 2048])
+def test_sparse_limits_agree(layer, limit):
+    """A batch at a limit and one token above it: the shared rows agree (the
+    kernels differ in the order of their fp32 sums only)."""
+    L, _ = layer
+    x = synth.inputs(530, limit + 1, L.spec.width)
+    a, b = P.forward(L, x[:limit]), P.forward(L, x)
+    np.testing.assert_array_equal(a.ids.get()[:limit], b.ids.get()[:limit])
+    u, v = a.out.get()[:limit].astype(np.float64), b.out.get()[:limit].astype(np.float64)
+    rel = np.linalg.norm(u - v) / np.linalg.norm(v)
+    print(f"limit {limit} D={L.spec.width}: rel {rel:.2e}", flush=True, file=sys.stderr)
+    assert rel < 3e-6  # each within 7e-7 of the 64-bit result
+
+
+def test_sparse_all_tokens_handed_off(layer):
+    """No expert resident and a zero threshold: every token is flagged, so the
+    routed groups are all empty and only the shared expert (or nothing) runs."""
+    from nebula_amd import qg
+    L, H = layer
+    nt = 40
+    desc = qg.MoeLayer.from_buffer_copy(L.desc)
+    mask = qg.Device(np.zeros(512, np.uint8))
+    desc.resident, desc.threshold = mask.p, 0.10
+    saved, L.desc = L.desc, desc
+    try:
+        x = synth.inputs(540, nt, L.spec.width)
+        fw = P.forward(L, x)
+        flags = fw.flags.get()[:nt]
+        assert np.all(flags == 2)
+        got = fw.out.get()[:nt]
+        if H.shared:
+            P.assert_close(got, H.shared_part(x), "shared part alone")
+        else:
+            assert np.all(got == 0)
+    finally:
+        L.desc = saved
