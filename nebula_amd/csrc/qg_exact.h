@@ -14,21 +14,6 @@
 
 typedef float qg_f16v __attribute__((ext_vector_type(16)));
 
-// Direct global->shared copy of 16 bytes per lane from base + off (bytes),
-// issued from inline assembly as dma16_ordered is: lane l's data lands at
-// lds_base + 16 l.
-QG_DEV void xm_copy16(uint32_t off, const void *base, void *lds_base) {
-    const uint32_t b = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(qg_lds_void *)lds_base);
-    const uint64_t g = (uint64_t)base;  // uniform: kept in scalar registers
-    const uint32_t g_lo = __builtin_amdgcn_readfirstlane((uint32_t)g), g_hi = __builtin_amdgcn_readfirstlane((uint32_t)(g >> 32));
-    const uint64_t sg = (uint64_t)g_hi << 32 | g_lo;
-    uint32_t saved;
-    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-                 : "=&s"(saved)
-                 : "v"(off), "s"(sg), "s"(b)
-                 : "memory");
-}
-
 // A tile is TOK = 16 N16 + 4 N4 tokens x 16 RR weight rows; K streams in
 // stages of CH chunks of 128 columns (4 steps of every chain).  The
 // workgroup's 8 waves split the chains: wave w owns chains 2w, 2w + 1, 2w +
@@ -120,10 +105,10 @@ __global__ __launch_bounds__(512, OCC) void xm_kernel(XmArgs A) {
 #pragma unroll
             for (int i = 0; i < NX; i++)
                 if (64 * (i + 1) <= 4 * TOK || lane < 4 * TOK - 64 * i)
-                    xm_copy16(xo[i], xb + (size_t)(cc * CH + q) * 512, xs + (slot * CH + q) * (TOK * 128) + 4 * (4 * TOK * wave + 64 * i));
+                    dma16_scalar(xo[i], xb + (size_t)(cc * CH + q) * 512, xs + (slot * CH + q) * (TOK * 128) + 4 * (4 * TOK * wave + 64 * i));
 #pragma unroll
             for (int i = 0; i < NW; i++)
-                xm_copy16(wo[i], wb + (size_t)(cc * CH + q) * 512, ws + (slot * CH + q) * (ROWS * 128) + 4 * (4 * ROWS * wave + 64 * i));
+                dma16_scalar(wo[i], wb + (size_t)(cc * CH + q) * 512, ws + (slot * CH + q) * (ROWS * 128) + 4 * (4 * ROWS * wave + 64 * i));
         }
     };
     // raw superblock s: the wave's rows v (row 16 (v / 2) + 2 wave + v % 2)
@@ -135,7 +120,7 @@ __global__ __launch_bounds__(512, OCC) void xm_kernel(XmArgs A) {
     }
     auto copy_raw = [&](int s) {
         if constexpr (RB != 0) {
-            if (lane < S::WROWS * PC) xm_copy16(ro, wb + (size_t)min(s, nsb - 1) * RB, raw + (s % RS) * S::RAW + wave * (S::WROWS * RB));
+            if (lane < S::WROWS * PC) dma16_scalar(ro, wb + (size_t)min(s, nsb - 1) * RB, raw + (s % RS) * S::RAW + wave * (S::WROWS * RB));
         }
     };
     // the scales of the wave's rows in superblock s

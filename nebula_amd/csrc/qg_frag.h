@@ -193,6 +193,18 @@ QG_DEV void dma4_ordered(const void *g, void *lds_base) {
                  : "v"(g), "s"(base)
                  : "memory");
 }
+// dma16_ordered from base + off (bytes), base uniform across the wave.
+QG_DEV void dma16_scalar(uint32_t off, const void *base, void *lds_base) {
+    const uint32_t b = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(qg_lds_void *)lds_base);
+    const uint64_t g = (uint64_t)base;  // uniform: kept in scalar registers
+    const uint32_t g_lo = __builtin_amdgcn_readfirstlane((uint32_t)g), g_hi = __builtin_amdgcn_readfirstlane((uint32_t)(g >> 32));
+    const uint64_t sg = (uint64_t)g_hi << 32 | g_lo;
+    uint32_t saved;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
+                 : "=&s"(saved)
+                 : "v"(off), "s"(sg), "s"(b)
+                 : "memory");
+}
 QG_DEV void wait_vmem() { __builtin_amdgcn_s_waitcnt(0); }
 // Wait until at most N vector-memory operations of this wave are outstanding
 // (they complete in issue order), leaving the other counters alone.

@@ -172,14 +172,22 @@ QG_DEV void sp_pin(qg_half8 &f) {
 // ---- gate/up: K split over the waves ----
 // Wave w (of W = D / 256) multiplies superblock w of a sub-unit's 16 gate and 16
 // up rows (144 bytes each, copied two sub-units ahead into the wave's ring of
-// three slots, row r's 9 pieces rotated by r / 8 for the banks); partial sums
-// meet in shared memory and 2 T waves apply SwiGLU.  A unit is 32 F rows (two
-// sub-units), the group of a Q4_K down's min term.
+// three slots, row r's 9 pieces rotated by r / 8 for the banks).  The partial
+// sums of up to NB sub-units meet in shared memory before a barrier, after
+// which 2 T waves per sub-unit apply SwiGLU, so that with one tile the products
+// of four sub-units run without a barrier and every wave has a share of their
+// epilogue.  A unit is 32 F rows (two sub-units), the group of a Q4_K down's
+// min term.
 constexpr int SP_SLOT = 32 * 9;     // 16-byte pieces of a sub-unit's rows per wave
-constexpr int SP_CPB = 5;           // copies per sub-unit and wave
+constexpr int SP_CPB = 6;           // copies per sub-unit and wave
 template <int W, int TM> struct SpGu {
-    static constexpr int RING = W * 3 * SP_SLOT * 16, RED = W * 2 * TM * 64 * 8, LDS = RING + RED;
-    static_assert(W >= 2 * TM, "a wave per tile and token of a lane pair");
+    // tile slots of the partial sums: what 160 KB leave beside the rings
+    static constexpr int TS = W == 8 ? 6 : 2;
+    static constexpr int RING = W * 3 * SP_SLOT * 16, RED = W * 2 * TS * 64 * 8, LDS = RING + RED;
+    static_assert(W >= 2 * TM && TS >= TM, "a wave per tile and token of a lane pair");
+    // sub-units per barrier with M tiles
+    static constexpr int batch(int M) { return min_(min_(4, TS) / M, W / (2 * M)) > 0 ? min_(min_(4, TS) / M, W / (2 * M)) : 1; }
+    static constexpr int min_(int a, int b) { return a < b ? a : b; }
 };
 
 struct SpGuArgs {
@@ -196,6 +204,7 @@ __global__ __launch_bounds__(64 * W, 1) void pf_gateup_sp_kernel(SpGuArgs A) {
     extern __shared__ uint4 s_dyn[];
     __shared__ SpList S;
     __shared__ int s_off[QG_EXPERTS + 1];
+    __shared__ float s_gs[W][4];   // 16-row sums of the jobs' tile rows (Q4_K down format)
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, j = lane & 15, kq = lane >> 4;
     for (int i = tid; i <= QG_EXPERTS; i += 64 * W) s_off[i] = A.offsets[i];
     __syncthreads();
@@ -206,42 +215,42 @@ __global__ __launch_bounds__(64 * W, 1) void pf_gateup_sp_kernel(SpGuArgs A) {
     uint4 *ring = s_dyn + (size_t)wave * 3 * SP_SLOT;
     float2 *red = (float2 *)(s_dyn + SpGu<W, TM>::RING / 16);
 
-    // copies: piece 64 i + lane of a slot; copies 0..3 go out under one M0
-    // value whose instruction offsets move the global address too
-    uint32_t c_off[SP_CPB];
-    bool c_up[SP_CPB];
+    // copies: piece 64 i + lane of a slot, at c_off[i] from its matrix's first
+    // row of the sub-unit; pieces 0..143 are gate rows, the others up rows, so
+    // piece run 2 goes out as two copies of 16 and 48 lanes
+    uint32_t c_off[5];
 #pragma unroll
-    for (int i = 0; i < SP_CPB; i++) {
+    for (int i = 0; i < 5; i++) {
         const int sl = min(i * 64 + lane, SP_SLOT - 1), row = sl / 9, pc = sl - 9 * row, rot = row >> 3;
         c_off[i] = (uint32_t)((row & 15) * A.rb) + (uint32_t)(wave * 144 + 16 * (pc - rot + (pc < rot ? 9 : 0)));
-        c_up[i] = row >= 16;
     }
     int cx = __builtin_amdgcn_readfirstlane(S.pos[0][0]), ctau = __builtin_amdgcn_readfirstlane(S.pos[0][1]);
     int csub = 2 * __builtin_amdgcn_readfirstlane(S.pos[0][2]), cruns = 0;
     int x = cx, tau = ctau, sub = csub;
-    const uint8_t *cp[SP_CPB];
+    const uint8_t *bg = nullptr, *bu = nullptr;   // gate and up rows of the sub-unit to copy next
     auto set_copy = [&]() {
         const SpItem it = sp_item<TM>(S, s_off, A.nt, cx, ctau);
         cruns = it.runs;
         const bool sh = it.e == QG_EXPERTS;
         const size_t at = (size_t)csub * 16 * A.rb;
-        const uint8_t *bg = (sh ? A.sh_gate : A.gate + (size_t)it.e * F * A.rb) + at;
-        const uint8_t *bu = (sh ? A.sh_up : A.up + (size_t)it.e * F * A.rb) + at;
-#pragma unroll
-        for (int i = 0; i < SP_CPB; i++) cp[i] = (c_up[i] ? bu : bg) + c_off[i];
+        bg = (sh ? A.sh_gate : A.gate + (size_t)it.e * F * A.rb) + at;
+        bu = (sh ? A.sh_up : A.up + (size_t)it.e * F * A.rb) + at;
     };
     auto copy_next = [&](int slot) {
         uint4 *dst = ring + slot * SP_SLOT;
-        dma16x3_ordered(cp[0], cp[1], cp[2], dst);
-        dma16_ordered(cp[3], dst + 192);
-        if (lane < SP_SLOT - 256) dma16_ordered(cp[4], dst + 256);
+        dma16_scalar(c_off[0], bg, dst);
+        dma16_scalar(c_off[1], bg, dst + 64);
+        if (lane < 16) dma16_scalar(c_off[2], bg, dst + 128);
+        else dma16_scalar(c_off[2], bu, dst + 128);
+        dma16_scalar(c_off[3], bu, dst + 192);
+        if (lane < SP_SLOT - 256) dma16_scalar(c_off[4], bu, dst + 256);
         if (++csub == nsr) {
             csub = 0;
             if (++ctau == cruns) { ctau = 0; cx++; }
             if (cx < __builtin_amdgcn_readfirstlane(S.nx)) set_copy();
         } else {
-#pragma unroll
-            for (int i = 0; i < SP_CPB; i++) cp[i] += 16 * A.rb;
+            bg += 16 * A.rb;
+            bu += 16 * A.rb;
         }
     };
     set_copy();
@@ -273,58 +282,71 @@ __global__ __launch_bounds__(64 * W, 1) void pf_gateup_sp_kernel(SpGuArgs A) {
             sp_pin(sf[m]);
         }
         const int fmt = sh ? A.sh_down_fmt : A.down_fmt;
-        float half = 0.0f;   // the first 16 rows' sum of the unit's 32-row group
-        for (int c = 0; c < cnt; c++, it++) {
-            if (it + 2 < nsub) copy_next(qc == 0 ? 2 : qc - 1);
-            if (it + 2 < nsub) wait_vmem_but<2 * SP_CPB>();
-            else if (it + 1 < nsub) wait_vmem_but<SP_CPB>();
-            else wait_vmem();
-            float2 y[2][M];
-            ksplit_products<M>(ring + qc * SP_SLOT, af, sf, j, kq, y);
-            qc = qc == 2 ? 0 : qc + 1;
-            __syncthreads();  // the previous sub-unit's sums have been read
+        constexpr int NB = SpGu<W, TM>::batch(M);
+        constexpr bool TWO = NB == 1 && SpGu<W, TM>::TS >= 2 * M;   // sub-units alternate between two sum buffers
+        float half = 0.0f;   // NB == 1: the first 16 rows' sum of the unit's 32-row group
+        __syncthreads();     // the previous run's sums have been read
+        for (int c = 0; c < cnt; c += NB) {
+            const int nb = min(NB, cnt - c);
+            float2 *rd = red + (TWO ? (c & 1) * (W * 2 * M * 64) : 0);
+            for (int b = 0; b < nb; b++, it++) {
+                if (it + 2 < nsub) copy_next(qc == 0 ? 2 : qc - 1);
+                if (it + 2 < nsub) wait_vmem_but<2 * SP_CPB>();
+                else if (it + 1 < nsub) wait_vmem_but<SP_CPB>();
+                else wait_vmem();
+                float2 y[2][M];
+                ksplit_products<M>(ring + qc * SP_SLOT, af, sf, j, kq, y);
+                qc = qc == 2 ? 0 : qc + 1;
 #pragma unroll
-            for (int cb = 0; cb < 2; cb++)
+                for (int cb = 0; cb < 2; cb++)
 #pragma unroll
-                for (int m = 0; m < M; m++) red[((wave * 2 + cb) * TM + m) * 64 + lane] = y[cb][m];
+                    for (int m = 0; m < M; m++) rd[(((b * M + m) * 2 + cb) * W + wave) * 64 + lane] = y[cb][m];
+            }
             __syncthreads();
-            if (wave < 2 * M) {
-                // tile m, row 2 kq + t2 of it, F row j of the sub-unit
-                const int m = wave >> 1, t2 = wave & 1, idx = 8 * m + 2 * kq + t2;
+            // jobs: sub-unit b, tile m, row 2 kq + t2 of it; F row j
+            const int b = wave / (2 * M), m = (wave % (2 * M)) >> 1, t2 = wave & 1, idx = 8 * m + 2 * kq + t2;
+            const int row = (sh ? A.nt * QG_TOP : 0) + R.base + idx;
+            float s16 = 0.0f;
+            if (b < nb) {
                 float g = 0.0f, u = 0.0f;
 #pragma unroll
                 for (int w = 0; w < W; w++) {
-                    const float2 ga = red[((w * 2 + 0) * TM + m) * 64 + lane], ua = red[((w * 2 + 1) * TM + m) * 64 + lane];
+                    const float2 ga = rd[(((b * M + m) * 2 + 0) * W + w) * 64 + lane], ua = rd[(((b * M + m) * 2 + 1) * W + w) * 64 + lane];
                     g += t2 ? ga.y : ga.x;
                     u += t2 ? ua.y : ua.x;
                 }
-                const int f = (sub + c) * 16 + j, pos = plane_pos(fmt, f);
-                const size_t row = (size_t)((sh ? A.nt * QG_TOP : 0) + R.base + idx);
+                const int pos = plane_pos(fmt, (sub + c + b) * 16 + j);
                 const float mv = qg_swiglu_fast(g, u);
                 if (idx < R.n) {
-                    _Float16 *mp = A.midp + row * 2 * F;
+                    _Float16 *mp = A.midp + (size_t)row * 2 * F;
                     const _Float16 hv = (_Float16)mv;
                     mp[pos] = hv;
                     mp[F + pos] = (_Float16)(mv - (float)hv);
                 }
                 if (fmt == QT_Q4_K) {
-                    float s = mv;
-                    s += __shfl_xor(s, 1);
-                    s += __shfl_xor(s, 2);
-                    s += __shfl_xor(s, 4);
-                    s += __shfl_xor(s, 8);
-                    if ((sub + c) & 1) {
-                        s += half;
-                        if (j == 0 && idx < R.n) {
-                            _Float16 *gp = A.msp + row * 2 * (F / 32) + ((sub + c) >> 1);
-                            const _Float16 hs = (_Float16)s;
-                            gp[0] = hs;
-                            gp[F / 32] = (_Float16)(s - (float)hs);
-                        }
-                    } else {
-                        half = s;
+                    s16 = mv;
+                    s16 += __shfl_xor(s16, 1);
+                    s16 += __shfl_xor(s16, 2);
+                    s16 += __shfl_xor(s16, 4);
+                    s16 += __shfl_xor(s16, 8);
+                    if (NB > 1 && j == 0) s_gs[wave][kq] = s16;
+                }
+            }
+            if (!TWO) __syncthreads();  // the sums have been read
+            if (fmt == QT_Q4_K && b < nb) {
+                // the odd sub-unit's job writes its group's sum (a batch
+                // starts and ends on even sub-units when NB > 1)
+                const int sb = sub + c + b;
+                if (sb & 1) {
+                    const float sum = s16 + (NB > 1 ? s_gs[wave >= 2 * M ? wave - 2 * M : 0][kq] : half);
+                    if (j == 0 && idx < R.n) {
+                        _Float16 *gp = A.msp + (size_t)row * 2 * (F / 32) + (sb >> 1);
+                        const _Float16 hs = (_Float16)sum;
+                        gp[0] = hs;
+                        gp[F / 32] = (_Float16)(sum - (float)hs);
                     }
                 }
+                half = s16;
             }
         }
     };
@@ -409,7 +431,7 @@ __global__ __launch_bounds__(512, 1) void pf_down_sp_kernel(SpDnArgs A) {
         const uint8_t *b = (CR.e == QG_EXPERTS ? A.sh_down : A.down + (size_t)CR.e * D * RB) + (size_t)cu * 16 * RB;
 #pragma unroll
         for (int i = 0; i < CP; i++)
-            if (64 * (i + 1) <= C::PCS || lane < C::PCS - 64 * i) dma16_ordered(b + c_off[i], ring + slot * C::SLOT + 1024 * i);
+            if (64 * (i + 1) <= C::PCS || lane < C::PCS - 64 * i) dma16_scalar(c_off[i], b, ring + slot * C::SLOT + 1024 * i);
         cu += 8;
         settle(cx, ctau, cu, CR);
     };
