@@ -38,8 +38,7 @@
 // activation rows (64 rows x 2 planes x one K step) are staged in shared
 // memory by direct global->shared copies, double-buffered over steps; each
 // wave owns 32 weight rows (gate/up: 16 gate + 16 up) whose quantised bytes
-// it copies, two steps ahead, into a ring of its own in shared memory (the
-// Q4_K down launch keeps them in registers instead).  A
+// it copies, two steps ahead, into a ring of its own in shared memory.  A
 // 16x16x32 MFMA pair (hi and lo plane) per (row tile, column tile, 32-element
 // group); row tiles past the group's last row are skipped.  16-byte chunk c of
 // a staged row r sits at chunk c ^ (r & 15), so the 16 rows one MFMA reads
@@ -56,14 +55,10 @@ namespace {
 constexpr int PF_MIN = QG_MAX_DECODE + 1;   // smallest batch on this path
 constexpr int PF_CHUNK = 32;                 // tokens per routing chunk (one 32-bit mask per expert)
 constexpr int PT = 64;                       // rows per GEMM tile
-constexpr int KC = 256;                      // K elements per staged chunk
 constexpr int GU_FB = 128;                   // F rows per gate/up item (16 per wave)
 constexpr int DN_DB = 256;                   // D rows per down item (32 per wave)
 constexpr int NG = QG_EXPERTS + 1;           // groups: experts + shared expert
 constexpr int DENSE_MIN = 256;               // rows from which an expert is dense (pass order; the int8 variant)
-constexpr int STAGE_BYTES = PT * 2 * KC * 2; // [64 rows][2 planes][256] fp16
-constexpr int SUMS_BYTES = PT * 2 * 16;      // [64 rows][2 planes][8 group sums] fp16
-constexpr int PF_LDS = 2 * (STAGE_BYTES + SUMS_BYTES);
 
 // Groups in pass order: the dense experts (>= DENSE_MIN rows), the shared
 // expert, the other experts; experts by row count, largest first (ties by
@@ -418,98 +413,6 @@ __global__ __launch_bounds__(512) void pf_fill_kernel(int *row_token, int *row_s
 constexpr int PF_WAVES = 8;                  // waves per GEMM workgroup
 constexpr int NCT = 2;                       // column tiles of 16 weight rows per wave
 
-// Stage K chunk `chunk` of the tile's first nrows rows (a multiple of 16):
-// plane rows of `planes` (row stride `stride` elements per plane, 2 planes
-// per source row; source row of tile row r = src[r]) into `stage`, swizzled;
-// nck = 16-byte chunks per plane row in this K chunk.  With `sums`, the 2 x 8
-// group sums of the chunk ([tile row][plane][8]).
-QG_DEV void stage_rows(uint8_t *stage, uint8_t *sums, const _Float16 *planes, int stride, const _Float16 *sum_planes,
-                       int sum_stride, const int *src, int chunk, int nck, int nrows, int wave, int lane) {
-    for (int q = wave; q < nrows; q += PF_WAVES) {
-        const int R = 2 * q + (lane >> 5), tr = R >> 1, p = R & 1;
-        int c = (lane & 31) ^ (tr & 15);
-        if (c >= nck) c = 0;  // positions no reader uses
-        dma16_ordered(planes + ((size_t)src[tr] * 2 + p) * stride + (size_t)chunk * KC + c * 8, stage + q * 1024);
-    }
-    if (sums && wave * 32 < nrows) {
-        const int C = wave * 64 + lane, tr = C >> 1, p = C & 1;
-        dma16_ordered(sum_planes + ((size_t)src[tr] * 2 + p) * sum_stride + (size_t)chunk * 8, sums + wave * 1024);
-    }
-}
-
-// A fragment of tile row r (within the stage), plane p, 16-byte chunk c.
-QG_DEV qg_half8 stage_frag(const uint8_t *st, int r, int p, int c) {
-    return ld_frag((const _Float16 *)(st + (r * 2 + p) * 512 + 16 * (c ^ (r & 15))));
-}
-
-// Q4_K operands of one superblock for the wave's column tiles: 3 loads per
-// tile (header, qs chunks kq and kq + 4).
-constexpr int Q4_LOADS = 3 * NCT;
-struct Q4Ops { uint4 hd[NCT], c0[NCT], c1[NCT]; };
-QG_DEV void q4_load(Q4Ops &o, const uint8_t *const *wrow, int sb, int kq) {
-#pragma unroll
-    for (int n = 0; n < NCT; n++) {
-        const uint8_t *p = wrow[n] + (size_t)sb * 144;
-        o.hd[n] = qg_ld16(p);
-        o.c0[n] = qg_ld16(p + 16 + 16 * kq);
-        o.c1[n] = qg_ld16(p + 16 + 16 * (kq + 4));
-    }
-}
-
-// y[m][n] += d * (s*q . x) - dmin * (m . X) over one Q4_K superblock, for the
-// first M row tiles (A fragments read from shared memory per K step; the
-// other wave on the SIMD hides their latency).
-QG_DEV void q4_chunk(qg_f4 (&y)[4][NCT], const Q4Ops &o, const uint8_t *st, const uint8_t *ss, int j, int kq, int M) {
-    Q4kHeader h[NCT];
-#pragma unroll
-    for (int n = 0; n < NCT; n++) h[n] = q4k_header(o.hd[n]);
-    qg_f4 acc[4][NCT];
-#pragma unroll
-    for (int m = 0; m < 4; m++)
-#pragma unroll
-        for (int n = 0; n < NCT; n++) acc[m][n] = qg_f4{0.0f, 0.0f, 0.0f, 0.0f};
-    const int gA = 2 * (kq >> 1);
-#pragma unroll
-    for (int f = 0; f < 8; f++) {
-        qg_half8 b[NCT];
-#pragma unroll
-        for (int n = 0; n < NCT; n++) {
-            const uint4 c = f < 4 ? o.c0[n] : o.c1[n];
-            const int g = (f < 4 ? gA : gA + 4) + ((f & 3) >> 1);
-            b[n] = q4k_chunk_frag(c, f & 3, (_Float16)q4k_s(h[n], g));
-        }
-#pragma unroll
-        for (int m = 0; m < 4; m++) {
-            if (m < M) {  // uniform
-                const qg_half8 a0 = stage_frag(st, m * 16 + j, 0, 4 * f + kq), a1 = stage_frag(st, m * 16 + j, 1, 4 * f + kq);
-#pragma unroll
-                for (int n = 0; n < NCT; n++) {
-                    acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a0, b[n], acc[m][n], 0, 0, 0);
-                    acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a1, b[n], acc[m][n], 0, 0, 0);
-                }
-            }
-        }
-    }
-    // min term: lanes kq = 0 / 1 carry the hi / lo plane of the 8 group sums
-    const qg_half8 z8 = qg_half8{0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-    for (int n = 0; n < NCT; n++) {
-        qg_half8 bm;
-#pragma unroll
-        for (int g = 0; g < 8; g++) bm[g] = kq < 2 ? (_Float16)q4k_m(h[n], g) : (_Float16)0.0f;
-#pragma unroll
-        for (int m = 0; m < 4; m++) {
-            if (m < M) {
-                const qg_half8 as = kq < 2 ? ld_frag((const _Float16 *)(ss + ((m * 16 + j) * 2 + kq) * 16)) : z8;
-                const qg_f4 mm = __builtin_amdgcn_mfma_f32_16x16x32_f16(as, bm, qg_f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    y[m][n][i] = __builtin_fmaf(h[n].d, acc[m][n][i], __builtin_fmaf(-h[n].dmin, mm[i], y[m][n][i]));
-            }
-        }
-    }
-}
-
 // Items of a persistent launch, XCD-aware: workgroup b runs on XCD b % 8
 // (round-robin dispatch) and takes its XCD's share xs .. xe-1 of the items
 // in rounds of nx (the XCD's workgroups), position slot of each round, so
@@ -633,10 +536,6 @@ QG_DEV void item_rows(int *dst, const PfItem &it, const int *list, int shared_ba
     else dma4_ordered(list + r, dst);
 }
 
-// Position (item k, chunk c) of a step, advanced without division.
-struct StepPos { int k, c; };
-QG_DEV StepPos next_pos(StepPos p, int nc) { return ++p.c == nc ? StepPos{p.k + 1, 0} : p; }
-
 // ---------------- P5: gate/up + SwiGLU ----------------
 struct GuArgs {
     int nt, D, F;
@@ -661,121 +560,6 @@ struct DnArgs {
     float *slots;                    // [rows][D]: slot t*10+k, shared rows at nt*10+t
 };
 
-// Q4_K down.  Item = (group, 64-row tile, 256 D rows); wave w: D rows 32 w ..
-// +31 of the block as two column tiles, their weights in registers loaded two
-// steps ahead.  Steps are the item's K chunks of 256 (F / 256 superblocks).
-__global__ __launch_bounds__(512, 1) void pf_down_kernel(DnArgs A) {
-    extern __shared__ uint4 s_dyn[];
-    uint8_t *lds = (uint8_t *)s_dyn;
-    __shared__ int s_tb[NG + 1], s_go[NG], s_off[QG_EXPERTS + 1];
-    __shared__ int2 s_it[IT_RING];
-    __shared__ int s_src[2][PT], s_slot[2][PT];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, kq = lane >> 4;
-    for (int i = tid; i <= NG; i += 512) {
-        s_tb[i] = A.tt->tbase[i];
-        if (i < NG) s_go[i] = A.tt->gorder[i];
-        if (i <= QG_EXPERTS) s_off[i] = A.offsets[i];
-    }
-    const int ndb = A.D / DN_DB, F = A.F, F32 = A.F / 32, nkc = (F + KC - 1) / KC;
-    const int t_lo = A.tt->bounds[A.seg_lo], total = (A.tt->bounds[A.seg_hi] - t_lo) * ndb;
-    const ItemRange ir = balanced_items<10, 3>(A.tt, s_tb, A.seg_lo, A.seg_hi, ndb);
-    const int nitems = range_count(ir), steps = nitems * nkc;
-    if (steps == 0) return;  // block-uniform
-    const ItemRing R{s_it, s_tb, s_go, s_off, A.nt, t_lo, ndb, nitems, ir};
-    __syncthreads();
-    R.fill(0, IT_RING, tid);
-    __syncthreads();
-    // the item's mid rows (computed) and output slots (copied from row_slot)
-    auto set_rows = [&](const PfItem &it, int buf) {
-        if (wave == 0) s_src[buf][lane] = (it.shared ? A.nt * QG_TOP : 0) + it.base + min(lane, it.nv - 1);
-        item_rows(s_slot[buf], it, A.row_slot, A.nt * QG_TOP, wave, lane);
-    };
-    auto weight_rows = [&](const PfItem &it, const uint8_t **wrow) {
-        const uint8_t *bw = it.shared ? A.sh_down : A.down + (size_t)it.g * A.D * A.rb;
-        const size_t rb = it.shared ? A.sh_rb : A.rb;
-        const int d = it.blk * DN_DB + wave * 32 + j;
-#pragma unroll
-        for (int n = 0; n < NCT; n++) wrow[n] = bw + (size_t)(d + 16 * n) * rb;
-    };
-    auto stage = [&](const PfItem &it, int buf, int kc, int b) {
-        stage_rows(lds + b * STAGE_BYTES, lds + 2 * STAGE_BYTES + b * SUMS_BYTES, A.midp, F, A.msp, F32, s_src[buf], kc, 32,
-                   16 * it.M, wave, lane);
-    };
-    using Ops = Q4Ops;
-    const uint8_t *wrow[NCT];
-    auto load_step = [&](Ops &o, StepPos p) {
-        weight_rows(R.at(p.k), wrow);
-        q4_load(o, wrow, p.c, kq);
-    };
-    PfItem cur = R.at(0);
-    set_rows(cur, 0);
-    wait_vmem();
-    __syncthreads();
-    stage(cur, 0, 0, 0);
-    Ops w0, w1, w2;   // weights of step s in w[s % 3], loaded two steps ahead, never copied
-    StepPos pos{0, 0};
-    load_step(w0, pos);
-    if (1 < steps) load_step(w1, next_pos(pos, nkc));
-    qg_f4 y[4][NCT];
-#pragma unroll
-    for (int m = 0; m < 4; m++)
-#pragma unroll
-        for (int n = 0; n < NCT; n++) y[m][n] = qg_f4{0.0f, 0.0f, 0.0f, 0.0f};
-    auto step = [&](int s, const Ops &wc, Ops &wn) {
-        const int k = pos.k, kc = pos.c;
-        const StepPos p1 = next_pos(pos, nkc), p2 = next_pos(p1, nkc);
-        if (s + 1 < steps) wait_vmem_but<Q4_LOADS>();
-        else wait_vmem();
-        __syncthreads();
-        if (kc == 0) {
-            if (k > 0 && (k & (IT_BATCH - 1)) == 0) R.fill(k + IT_BATCH, IT_BATCH, tid);
-            // the next item's rows, copied while this item streams
-            if (k + 1 < nitems) set_rows(R.at(k + 1), (k + 1) & 1);
-        }
-        if (s + 1 < steps) {
-            if (p1.k != k) {
-                if (nkc == 1) {  // the rows were copied just above
-                    wait_vmem();
-                    __syncthreads();
-                }
-                stage(R.at(p1.k), p1.k & 1, p1.c, (s + 1) & 1);
-            } else {
-                stage(cur, k & 1, p1.c, (s + 1) & 1);
-            }
-        }
-        if (s + 2 < steps) load_step(wn, p2);
-        const uint8_t *st = lds + (s & 1) * STAGE_BYTES, *ss = lds + 2 * STAGE_BYTES + (s & 1) * SUMS_BYTES;
-        q4_chunk(y, wc, st, ss, j, kq, cur.M);
-        if (kc == nkc - 1) {
-            const int d0 = cur.blk * DN_DB + wave * 32;
-#pragma unroll
-            for (int m = 0; m < 4; m++) {
-                if (m >= cur.M) break;
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    const int tr = m * 16 + 4 * kq + i;
-                    if (tr < cur.nv) {
-                        float *o = A.slots + (size_t)s_slot[k & 1][tr] * A.D + d0 + j;
-#pragma unroll
-                        for (int n = 0; n < NCT; n++) o[16 * n] = y[m][n][i];
-                    }
-                }
-            }
-#pragma unroll
-            for (int m = 0; m < 4; m++)
-#pragma unroll
-                for (int n = 0; n < NCT; n++) y[m][n] = qg_f4{0.0f, 0.0f, 0.0f, 0.0f};
-            if (s + 1 < steps) cur = R.at(k + 1);
-        }
-        pos = p1;
-    };
-    for (int s = 0; s < steps; s += 3) {
-        step(s, w0, w2);
-        if (s + 1 < steps) step(s + 1, w1, w0);
-        if (s + 2 < steps) step(s + 2, w2, w1);
-    }
-}
-
 // ---- IQ4_NL down: the weights through each wave's own shared-memory ring ----
 // IQ4_NL rows are 18-byte blocks, so a lane's bytes of a block (its scale and
 // 4 qs bytes) are two or three narrow loads.  Here each wave instead copies
@@ -796,15 +580,6 @@ static_assert(32 * IQ_PIECES <= IQ_COPIES * 64, "the copies cover the slot");
 
 // Activation stage of one 128-element K chunk: [row][plane][16 chunks of 16
 // bytes], chunk position c ^ (row & 15); one copy covers two rows.
-QG_DEV void stage_rows128(uint8_t *stage, const _Float16 *planes, int stride, const int *src, int chunk, int nck, int nrows,
-                          int wave, int lane) {
-    for (int q = wave; 2 * q < nrows; q += PF_WAVES) {
-        const int tr = 2 * q + (lane >> 5), p = (lane >> 4) & 1;
-        int c = (lane & 15) ^ (tr & 15);
-        if (c >= nck) c = 0;  // positions no reader uses
-        dma16_ordered(planes + ((size_t)src[tr] * 2 + p) * stride + (size_t)chunk * IQ_KC + c * 8, stage + q * 1024);
-    }
-}
 QG_DEV qg_half8 stage_frag128(const uint8_t *st, int r, int p, int c) {
     return ld_frag((const _Float16 *)(st + (r * 2 + p) * 256 + 16 * (c ^ (r & 15))));
 }
@@ -1049,13 +824,6 @@ static_assert(32 * GQ_PIECES <= GQ_COPIES * 64, "the copies cover the slot");
 // The int8 variant's stage of one 128-element K chunk: [row][plane][8 chunks
 // of 16 bytes] (natural K order), chunk position c ^ (row & 7); one copy
 // covers four rows.
-QG_DEV void stage_rows128_i8(uint8_t *stage, const int8_t *planes, int D, const int *src, int chunk, int nrows, int wave,
-                             int lane) {
-    for (int q = wave; 4 * q < nrows; q += PF_WAVES) {
-        const int tr = 4 * q + (lane >> 4), p = (lane >> 3) & 1, c = (lane & 7) ^ (tr & 7);
-        dma16_ordered(planes + ((size_t)src[tr] * 2 + p) * D + (size_t)chunk * 128 + c * 16, stage + q * 1024);
-    }
-}
 // 8 int8 activations of row r, plane p: elements 8 kq .. 8 kq + 7 of group f
 // of the chunk.
 QG_DEV long stage_frag128_i8(const uint8_t *st, int r, int p, int f, int kq) {
@@ -1410,6 +1178,153 @@ __global__ __launch_bounds__(512, 1) void pf_gateup_kernel(GuArgs A) {
     }
 }
 
+// Q4_K down over half-superblock steps, as the gate/up kernel: item = (group,
+// 64-row tile, 256 D rows); wave w: D rows 32 w .. +31 of the block as two column
+// tiles, their bytes through the wave's own ring; the mid rows (CSR order) staged
+// by direct copies, double-buffered; the step loop inside one instantiation per
+// row-tile count.  Against the kernel this replaces (weights in registers, a
+// test per row tile, 256-column steps): 698 -> 540 us at 8192
+// tokens (F 512), 59 -> 49 at 1500 (F 256).
+__global__ __launch_bounds__(512, 1) void pf_down_kernel(DnArgs A) {
+    extern __shared__ uint4 s_dyn[];
+    uint8_t *lds = (uint8_t *)s_dyn;
+    __shared__ int s_tb[NG + 1], s_go[NG], s_off[QG_EXPERTS + 1];
+    __shared__ int2 s_it[IT_RING];
+    __shared__ int s_slot[2][PT];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, kq = lane >> 4;
+    for (int i = tid; i <= NG; i += 512) {
+        s_tb[i] = A.tt->tbase[i];
+        if (i < NG) s_go[i] = A.tt->gorder[i];
+        if (i <= QG_EXPERTS) s_off[i] = A.offsets[i];
+    }
+    const int ndb = A.D / DN_DB, F = A.F, F32 = F / 32, NH = F / 128;   // NH steps per item (even)
+    const int t_lo = A.tt->bounds[A.seg_lo];
+    const ItemRange ir = balanced_items<7, 3>(A.tt, s_tb, A.seg_lo, A.seg_hi, ndb);
+    const int nitems = range_count(ir), steps = nitems * NH;
+    if (steps == 0) return;  // block-uniform
+    const ItemRing R{s_it, s_tb, s_go, s_off, A.nt, t_lo, ndb, nitems, ir};
+    __syncthreads();
+    R.fill(0, IT_RING, tid);
+    __syncthreads();
+    uint8_t *sums = lds + 2 * IQ_STAGE;                                             // two superblock sum buffers
+    uint8_t *ring = lds + 2 * IQ_STAGE + 2 * GQ_SUMS + (size_t)wave * 3 * GQ_SLOT;  // this wave's three slots
+    auto mrow = [&](const PfItem &it, int tr) { return (it.shared ? A.nt * QG_TOP : 0) + it.base + min(tr, it.nv - 1); };
+    auto set_rows = [&](const PfItem &it, int buf) { item_rows(s_slot[buf], it, A.row_slot, A.nt * QG_TOP, wave, lane); };
+    // weight copies: piece 64 t + lane of a slot is piece p of the wave's row r
+    // (the superblock's header or 16-byte piece p - 1 of the half's qs bytes)
+    uint32_t w_p[GQ_COPIES], w_r[GQ_COPIES], w_h[GQ_COPIES];
+#pragma unroll
+    for (int t = 0; t < GQ_COPIES; t++) {
+        const int i = min(t * 64 + lane, 32 * GQ_PIECES - 1), r = i / GQ_PIECES, p = i - GQ_PIECES * r;
+        w_r[t] = (uint32_t)r;
+        w_p[t] = (uint32_t)(16 * p);
+        w_h[t] = p == 0 ? 0u : 64u;
+    }
+    const uint8_t *wp[GQ_COPIES];  // the lane's rows of the item being copied
+    auto set_wp = [&](const PfItem &it) {
+        const size_t rb = it.shared ? A.sh_rb : A.rb;
+        const uint8_t *b = (it.shared ? A.sh_down : A.down + (size_t)it.g * A.D * A.rb) + (size_t)(it.blk * DN_DB + wave * 32) * rb;
+#pragma unroll
+        for (int t = 0; t < GQ_COPIES; t++) wp[t] = b + w_r[t] * rb + w_p[t];
+    };
+    auto copy_w = [&](int q, int c) {  // step c of the item being copied into slot q
+        const uint32_t sb = (uint32_t)(c >> 1) * 144u;
+        const bool h = c & 1;
+        static_assert(GQ_COPIES == 3, "three copies under one M0 value");
+        dma16x3_ordered(wp[0] + sb + (h ? w_h[0] : 0u), wp[1] + sb + (h ? w_h[1] : 0u), wp[2] + sb + (h ? w_h[2] : 0u),
+                        ring + q * GQ_SLOT);
+    };
+    // mid-plane copies of the item being staged: copy i of this wave covers tile
+    // rows 2 q, 2 q + 1 (q = wave + 8 i), and the rows' group sums
+    const uint8_t *sp[4] = {nullptr, nullptr, nullptr, nullptr}, *sump = nullptr;
+    int s_nc = 0;
+    bool s_sum = false;
+    auto set_sp = [&](const PfItem &it) {
+        s_nc = it.M;
+        s_sum = wave * 32 < 16 * it.M;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int tr = 2 * (wave + PF_WAVES * i) + (lane >> 5), p = (lane >> 4) & 1, c16 = (lane & 15) ^ (tr & 15);
+            if (i < it.M) sp[i] = (const uint8_t *)(A.midp + ((size_t)mrow(it, tr) * 2 + p) * F + c16 * 8);
+        }
+        if (s_sum) {
+            const int C = wave * 64 + lane, tr = C >> 1, p = C & 1;
+            sump = (const uint8_t *)(A.msp + ((size_t)mrow(it, tr) * 2 + p) * F32);
+        }
+    };
+    auto stage_at = [&](int s, int c) {  // the stage of step s (chunk c of the item being staged)
+        uint8_t *st = lds + (s & 1) * IQ_STAGE;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (i < s_nc) dma16_ordered(sp[i] + (size_t)c * 256, st + (wave + PF_WAVES * i) * 1024);
+        if ((c & 1) == 0 && s_sum) dma16_ordered(sump + (size_t)(c >> 1) * 16, sums + ((s >> 1) & 1) * GQ_SUMS + wave * 1024);
+    };
+    PfItem first = R.at(0);
+    set_rows(first, 0);
+    set_sp(first);
+    stage_at(0, 0);
+    set_wp(first);
+    copy_w(0, 0);
+    copy_w(1, 1);  // NH >= 2: step 1 is item 0's
+    int s = 0, qc = 0;  // step s reads slot s % 3; the copies of step s + 2 go to slot (s + 2) % 3 (read by step s - 1)
+    auto run_item = [&](const int k, auto MC) {
+        constexpr int M = decltype(MC)::value;
+        qg_f4 y[M][NCT];
+#pragma unroll
+        for (int m = 0; m < M; m++)
+#pragma unroll
+            for (int n = 0; n < NCT; n++) y[m][n] = qg_f4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int c = 0; c < NH; c++, s++) {
+            const int qn = qc == 0 ? 2 : qc - 1;
+            if (s + 1 < steps) wait_vmem_but<GQ_COPIES>();
+            else wait_vmem();
+            __syncthreads();
+            if (c == 0) {
+                if (k > 0 && (k & (IT_BATCH - 1)) == 0) R.fill(k + IT_BATCH, IT_BATCH, tid);
+                // the next item's slots (its buffer held item k - 1's, stored long ago)
+                if (k + 1 < nitems) set_rows(R.at(k + 1), (k + 1) & 1);
+            }
+            // the next step's stage, then the weights of step s + 2 (the wait
+            // above relies on this order), between the first K steps' products
+            auto issue = [&](int f) {
+                if (f == 0 && s + 1 < steps) {
+                    if (c == NH - 1) set_sp(R.at(k + 1));
+                    stage_at(s + 1, c == NH - 1 ? 0 : c + 1);
+                }
+                if (f == 1 && s + 2 < steps) {
+                    if (c == NH - 2) set_wp(R.at(k + 1));
+                    copy_w(qn, c + 2 < NH ? c + 2 : c + 2 - NH);
+                }
+            };
+            const uint8_t *ss = (c & 1) == 0 ? sums + ((s >> 1) & 1) * GQ_SUMS : nullptr;
+            gq_chunk<M, NCT, GQ_ROWB, 16>(y, ring + qc * GQ_SLOT, lds + (s & 1) * IQ_STAGE, ss, c & 1, j, kq, issue);
+            qc = qc == 2 ? 0 : qc + 1;
+        }
+        const PfItem it = R.at(k);
+        const int d0 = it.blk * DN_DB + wave * 32;
+#pragma unroll
+        for (int m = 0; m < M; m++) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int tr = m * 16 + 4 * kq + i;
+                if (tr < it.nv) {
+                    float *o = A.slots + (size_t)s_slot[k & 1][tr] * A.D + d0 + j;
+#pragma unroll
+                    for (int n = 0; n < NCT; n++) o[16 * n] = y[m][n][i];
+                }
+            }
+        }
+    };
+    for (int k = 0; k < nitems; k++) {
+        switch (R.at(k).M) {  // block-uniform
+        case 1: run_item(k, std::integral_constant<int, 1>{}); break;
+        case 2: run_item(k, std::integral_constant<int, 2>{}); break;
+        case 3: run_item(k, std::integral_constant<int, 3>{}); break;
+        default: run_item(k, std::integral_constant<int, 4>{}); break;
+        }
+    }
+}
+
 // The kernels of qg_sparse.h for batches whose experts have few rows, where
 // they stream and convert the weights in fewer instructions; above, the 64-row
 // tiles of pf_gateup_kernel and the down kernels re-read no weights.  The batch
@@ -1417,10 +1332,11 @@ __global__ __launch_bounds__(512, 1) void pf_gateup_kernel(GuArgs A) {
 //   gate/up D 2048: 40 tokens 111 / 67, 400 194 / 144, 1000 245 / 204, 1500 284 / 300
 //           D 2560: 60 tokens 200 / 147, 301 283 / 221, 600 297 / 271, 1200 366 / 471
 //           D 1024: 100 tokens 54 / 37, 600 66 / 53, 1500 80 / 97
-//   down Q4_K   F 512: 40 tokens 73 / 39, 600 136 / 93, 1500 189 / 170, 2500 249 / 260
-//        IQ4_NL F 512: 40 tokens 71 / 48, 400 129 / 116, 800 145 / 193
-//        IQ4_NL F 640: 60 tokens 131 / 89, 301 185 / 143, 600 197 / 233
-//        F 256, Q4_K: 1500 tokens 60 / 64; IQ4_NL: 100 tokens 35 / 28, 600 45 / 41, 1500 59 / 76
+//   down Q4_K   F 512: 200 tokens 108 / 74, 800 123 / 108, 1200 146 / 142
+//               F 256: 300 tokens 34 / 26, 600 39 / 35, 1000 42 / 48
+//        IQ4_NL F 512: 40 tokens 71 / 48, 400 127 / 117, 500 127 / 129
+//               F 640: 60 tokens 131 / 89, 301 185 / 139, 400 184 / 170, 600 197 / 233
+//               F 256: 100 tokens 35 / 28, 600 45 / 41, 1500 59 / 76
 // Runs of two tiles hold the mid fragments of K = 512 in registers for Q4_K; the
 // IQ4_NL conversion needs the registers, so it takes one tile there (with two,
 // spills in the loop made 400 tokens 262 us).
@@ -1443,8 +1359,8 @@ bool pf_down_sp(const SpDnArgs &A, int fmt, int F, int cus, hipStream_t s) {
     using N8 = std::integral_constant<int, 8>;
     using N16 = std::integral_constant<int, 16>;
     using N20 = std::integral_constant<int, 20>;
-    if (fmt == QT_Q4_K) return F == 256 ? go(Q4{}, N8{}, 1280) : F == 512 ? go(Q4{}, N16{}, 2048) : false;
-    return F == 256 ? go(IQ{}, N8{}, 640) : F == 512 ? go(IQ{}, N16{}, 448) : F == 640 ? go(IQ{}, N20{}, 400) : false;
+    if (fmt == QT_Q4_K) return F == 256 ? go(Q4{}, N8{}, 768) : F == 512 ? go(Q4{}, N16{}, 1280) : false;
+    return F == 256 ? go(IQ{}, N8{}, 640) : F == 512 ? go(IQ{}, N16{}, 448) : F == 640 ? go(IQ{}, N20{}, 448) : false;
 }
 
 // ---------------- P7: combine ----------------
@@ -1631,7 +1547,7 @@ int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsig
     auto down = [&](int seg_lo, int seg_hi, int fmt, int slot) {
         DnArgs DA{nt, D, F, offsets, tt, seg_lo, seg_hi, row_slot, (const uint8_t *)L->down, sh ? (const uint8_t *)L->sh_down : nullptr,
                   qg_row_bytes_host(L->down_type, F), sh ? qg_row_bytes_host(L->sh_down_type, F) : 0, midp, msp, slots};
-        if (fmt == QT_Q4_K) pf_launch(slot, pf_down_kernel, dim3(grid), dim3(512), PF_LDS, s, DA);
+        if (fmt == QT_Q4_K) pf_launch(slot, pf_down_kernel, dim3(grid), dim3(512), PF_GQ_LDS, s, DA);
         else pf_launch(slot, pf_down_iq_kernel, dim3(grid), dim3(512), PF_IQ_LDS, s, DA);
         return hipGetLastError();
     };

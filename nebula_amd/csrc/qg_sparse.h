@@ -499,7 +499,7 @@ __global__ __launch_bounds__(512, 1) void pf_down_sp_kernel(SpDnArgs A) {
 #pragma unroll
                         for (int i = 0; i < 4; i++) y[m][i] = __builtin_fmaf(d, acc[i], y[m][i]);
                     }
-                    if (b & 1) __builtin_amdgcn_sched_barrier(0);  // two blocks' operands live at a time
+                    if ((b & 7) == 7) __builtin_amdgcn_sched_barrier(0);  // eight blocks' operands live at a time
                 }
             } else {
 #pragma unroll

@@ -53,7 +53,7 @@ def test_sparse_short_groups(layer, nt):
     P.check_outputs(fw, L, H, x, P.sample_rows(nt, 8, nt), f"short groups D={L.spec.width} nt={nt}")
 
 
-@pytest.mark.parametrize("limit", [400, 448, 640, 896, 1280, 2048])
+@pytest.mark.parametrize("limit", [448, 640, 768, 896, 1280])
 def test_sparse_limits_agree(layer, limit):
     """A batch at a limit and one token above it: the shared rows agree (the
     kernels differ in the order of their fp32 sums only)."""
