@@ -1861,7 +1861,11 @@ size_t qg_moe_workspace_bytes(int width, int ff, int tokens) {
     // the residual form keeps the normalised input and the layer output of the
     // generic path after its own workspace
     const size_t extra = 2 * (((size_t)MB * width * 4 + 255) & ~(size_t)255);
-    const size_t d = dec_layout(width, ff).total;
+    size_t d = dec_layout(width, ff).total;
+    if (qg_prefill_small_shape(width, ff)) {
+        const size_t p = qg_prefill_workspace_bytes(width, ff, tokens);
+        d = p > d ? p : d;
+    }
     return (g + extra > d ? g + extra : d);
 }
 
@@ -1879,7 +1883,8 @@ int qg_moe_forward(float *out, int *ids, float *weights, unsigned char *flags, q
     if (!out || !ids || !weights || !x || !workspace || ws_bytes < qg_moe_workspace_bytes(L->width, L->ff, nt) ||
         !al16(out) || !al16(x) || !al16(workspace))
         return hipErrorInvalidValue;
-    if (nt > MB) return qg_prefill_forward(out, nullptr, ids, weights, flags, stats, x, nullptr, 0, nt, L, workspace);
+    if (nt > MB || (!dec_ok(L) && qg_prefill_small_ok(L, nt)))
+        return qg_prefill_forward(out, nullptr, ids, weights, flags, stats, x, nullptr, 0, nt, L, workspace);
     if (!dec_ok(L)) return qg_generic_forward(out, ids, weights, flags, stats, x, nt, L, workspace, ws_bytes);
     return dec_forward(out, nullptr, ids, weights, flags, stats, x, nullptr, 0, nt, L, (uint8_t *)workspace);
 }
@@ -1908,7 +1913,8 @@ int qg_moe_forward_residual(float *h, int *ids, float *weights, unsigned char *f
     if (!h || !ids || !weights || !workspace || ws_bytes < qg_moe_workspace_bytes(L->width, L->ff, nt) || !al16(h) ||
         !al16(xn_out) || !al16(out) || !al16(workspace))
         return hipErrorInvalidValue;
-    if (nt > MB) return qg_prefill_forward(out, h, ids, weights, flags, stats, h, xn_out, 1, nt, L, workspace);
+    if (nt > MB || (!dec_ok(L) && qg_prefill_small_ok(L, nt)))
+        return qg_prefill_forward(out, h, ids, weights, flags, stats, h, xn_out, 1, nt, L, workspace);
     if (dec_ok(L)) return dec_forward(out, h, ids, weights, flags, stats, h, xn_out, 1, nt, L, (uint8_t *)workspace);
     // generic form: normalise into the workspace tail, run the layer, add
     const int D = L->width;

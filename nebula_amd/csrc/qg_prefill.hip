@@ -52,7 +52,6 @@
 
 namespace {
 
-constexpr int PF_MIN = QG_MAX_DECODE + 1;   // smallest batch on this path
 constexpr int PF_CHUNK = 32;                 // tokens per routing chunk (one 32-bit mask per expert)
 constexpr int PT = 64;                       // rows per GEMM tile
 constexpr int GU_FB = 128;                   // F rows per gate/up item (16 per wave)
@@ -236,44 +235,12 @@ QG_DEV int scan512(int v, int *s_tmp) {
     return v + base;
 }
 
-// tt may be null (dispatch only); with `status`, *status = OR of bad[0..nch).
-__global__ __launch_bounds__(512) void pf_scan_kernel(int *counts, int nch, int *offsets, TileTable *tt, int shared_rows,
-                                                      const int *bad, int *status) {
-    __shared__ int s_tmp[8];
+// The tile table of experts with n rows each (thread e: expert e; a 512-thread
+// block).
+QG_DEV void tile_table(TileTable *tt, int n, int shared_rows, int *s_tmp) {
     __shared__ int s_tiles[NG], s_m16[NG];
     __shared__ int s_wh[8][64], s_above[64];
     const int e = threadIdx.x;
-    if (status) {
-        int b = 0;
-        for (int c = e; c < nch; c += QG_EXPERTS) b |= bad[c];
-        b = __syncthreads_or(b);
-        if (e == 0) *status = b ? 1 : 0;
-    }
-    constexpr int U = 16;  // loads in flight per thread
-    int n = 0;
-    for (int c0 = 0; c0 < nch; c0 += U) {
-        int v[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) v[u] = c0 + u < nch ? counts[(size_t)(c0 + u) * QG_EXPERTS + e] : 0;
-#pragma unroll
-        for (int u = 0; u < U; u++) n += v[u];
-    }
-    const int incl = scan512(n, s_tmp), off = incl - n;
-    offsets[e] = off;
-    if (e == QG_EXPERTS - 1) offsets[QG_EXPERTS] = incl;
-    // counts[c][e] -> first CSR position of chunk c's rows of expert e
-    int run = off;
-    for (int c0 = 0; c0 < nch; c0 += U) {
-        int v[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) v[u] = c0 + u < nch ? counts[(size_t)(c0 + u) * QG_EXPERTS + e] : 0;
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            if (c0 + u < nch) counts[(size_t)(c0 + u) * QG_EXPERTS + e] = run;
-            run += v[u];
-        }
-    }
-    if (!tt) return;  // block-uniform
     // pass order: experts by row-count bucket, largest first, ties by id (a
     // counting sort); buckets 0..16 hold ceil(n / 16) of the others, 17..63
     // the dense experts by 32-row steps, so the dense ones lead; the shared
@@ -352,6 +319,45 @@ __global__ __launch_bounds__(512) void pf_scan_kernel(int *counts, int nch, int 
     }
 }
 
+// tt may be null (dispatch only); with `status`, *status = OR of bad[0..nch).
+__global__ __launch_bounds__(512) void pf_scan_kernel(int *counts, int nch, int *offsets, TileTable *tt, int shared_rows,
+                                                      const int *bad, int *status) {
+    __shared__ int s_tmp[8];
+    const int e = threadIdx.x;
+    if (status) {
+        int b = 0;
+        for (int c = e; c < nch; c += QG_EXPERTS) b |= bad[c];
+        b = __syncthreads_or(b);
+        if (e == 0) *status = b ? 1 : 0;
+    }
+    constexpr int U = 16;  // loads in flight per thread
+    int n = 0;
+    for (int c0 = 0; c0 < nch; c0 += U) {
+        int v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = c0 + u < nch ? counts[(size_t)(c0 + u) * QG_EXPERTS + e] : 0;
+#pragma unroll
+        for (int u = 0; u < U; u++) n += v[u];
+    }
+    const int incl = scan512(n, s_tmp), off = incl - n;
+    offsets[e] = off;
+    if (e == QG_EXPERTS - 1) offsets[QG_EXPERTS] = incl;
+    // counts[c][e] -> first CSR position of chunk c's rows of expert e
+    int run = off;
+    for (int c0 = 0; c0 < nch; c0 += U) {
+        int v[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = c0 + u < nch ? counts[(size_t)(c0 + u) * QG_EXPERTS + e] : 0;
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (c0 + u < nch) counts[(size_t)(c0 + u) * QG_EXPERTS + e] = run;
+            run += v[u];
+        }
+    }
+    if (!tt) return;  // block-uniform
+    tile_table(tt, n, shared_rows, s_tmp);
+}
+
 // Histogram of an ids array alone (qg_moe_dispatch): chunk masks as in
 // pf_route_kernel; bad[chunk] = 1 if an id is neither in [0,512) nor a pruned
 // encoding in [-513,-2], or a token lists an expert twice (the validation of
@@ -406,6 +412,59 @@ __global__ __launch_bounds__(512) void pf_fill_kernel(int *row_token, int *row_s
         row_slot[pos] = (t0 + tl) * QG_TOP + k;
         if (row_sx) row_sx[pos] = xsc[t0 + tl];
     }
+}
+
+// P2b, P3 and P4 of a batch of up to PD_MAX tokens in one workgroup: the chunk
+// masks stay in shared memory and a thread's selections in its registers, so
+// one launch (and one read of the ids) replaces three.  In a captured graph
+// the layer is 3.7 us shorter at 40 tokens, 4.4 at 100, 1.5 at 200; at 500 one
+// workgroup looping over the selections was 0.7 longer.
+constexpr int PD_MAX = 256;
+constexpr int PD_SEL = PD_MAX * QG_TOP / 512;   // selections per thread
+__global__ __launch_bounds__(512) void pf_dispatch_kernel(int *offsets, TileTable *tt, int shared_rows, int *row_token, int *row_slot,
+                                                          const int *ids, const int *flag, int nt, float *row_sx, const float *xsc) {
+    constexpr int NCH = PD_MAX / PF_CHUNK;
+    __shared__ uint32_t s_mask[NCH][QG_EXPERTS];
+    __shared__ uint16_t s_before[NCH][QG_EXPERTS];   // rows of the expert in the chunks before
+    __shared__ int s_tmp[8], s_off[QG_EXPERTS];
+    const int tid = threadIdx.x, sel = nt * QG_TOP;
+    int id[PD_SEL], f[PD_SEL];
+#pragma unroll
+    for (int u = 0; u < PD_SEL; u++) {
+        const int i = min(tid + 512 * u, sel - 1);
+        id[u] = ids[i];
+        f[u] = flag[i / QG_TOP];
+    }
+#pragma unroll
+    for (int c = 0; c < NCH; c++) s_mask[c][tid] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PD_SEL; u++) {
+        const int i = tid + 512 * u, t = i / QG_TOP;
+        if (!(i < sel && f[u] < 2 && id[u] >= 0 && id[u] < QG_EXPERTS)) id[u] = -1;
+        else atomicOr(&s_mask[t / PF_CHUNK][id[u]], 1u << (t % PF_CHUNK));
+    }
+    __syncthreads();
+    int n = 0;
+#pragma unroll
+    for (int c = 0; c < NCH; c++) {
+        s_before[c][tid] = (uint16_t)n;
+        n += __popc(s_mask[c][tid]);
+    }
+    const int incl = scan512(n, s_tmp);
+    offsets[tid] = s_off[tid] = incl - n;
+    if (tid == QG_EXPERTS - 1) offsets[QG_EXPERTS] = incl;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PD_SEL; u++) {
+        if (id[u] < 0) continue;
+        const int i = tid + 512 * u, t = i / QG_TOP, c = t / PF_CHUNK;
+        const int pos = s_off[id[u]] + s_before[c][id[u]] + __popc(s_mask[c][id[u]] & ((1u << (t % PF_CHUNK)) - 1u));
+        row_token[pos] = t;
+        row_slot[pos] = i;
+        if (row_sx) row_sx[pos] = xsc[t];
+    }
+    if (tt) tile_table(tt, n, shared_rows, s_tmp);  // block-uniform
 }
 
 // ---------------- GEMM building blocks ----------------
@@ -1470,15 +1529,25 @@ bool qg_prefill_ok(const qg_moe_layer *L) {
 }
 
 size_t qg_prefill_workspace_bytes(int width, int ff, int tokens) {
-    if (width < 256 || width % DN_DB || width > 8192 || ff < GU_FB || ff % GU_FB || ff > 4096 || tokens < PF_MIN ||
+    if (width < 256 || width % DN_DB || width > 8192 || ff < GU_FB || ff % GU_FB || ff > 4096 || tokens < 1 ||
         tokens > QG_MAX_TOKENS)
         return 0;
     return pf_layout(width, ff, tokens).total;
 }
 
+// Decode batches at widths the decode kernels lack (2048 and 2560 are theirs),
+// for which both GEMM passes have a kernel of qg_sparse.h: the prefill path is
+// ahead of the generic kernels but for 2 and 3 tokens (1024/256, us per layer,
+// generic / prefill: 1 token 41.4 / 35.2, 2 36.5 / 37.1, 4 39.5 / 37.8, 8 55.8 /
+// 39.4, 17 75.9 / 44.2).
+bool qg_prefill_small_shape(int width, int ff) { return width == 1024 && (ff == 256 || ff == 512 || ff == 640); }
+bool qg_prefill_small_ok(const qg_moe_layer *L, int nt) {
+    return (nt == 1 || nt > 3) && qg_prefill_small_shape(L->width, L->ff) && qg_prefill_ok(L) && (!L->sh_gate || L->sh_down_type == L->down_type);
+}
+
 int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsigned char *flags, qg_prune_stats *stats,
                        const float *x, float *xn_out, int norm, int nt, const qg_moe_layer *L, void *workspace) {
-    if (nt < PF_MIN || nt > QG_MAX_TOKENS || !qg_prefill_ok(L)) return hipErrorInvalidValue;
+    if (nt < 1 || nt > QG_MAX_TOKENS || !qg_prefill_ok(L)) return hipErrorInvalidValue;
     const int D = L->width, F = L->ff;
     const PfLayout lay = pf_layout(D, F, nt);
     uint8_t *ws = (uint8_t *)workspace;
@@ -1514,14 +1583,20 @@ int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsig
                  sh ? L->sh_gate_inp : nullptr, logits + QG_EXPERTS, xi8, xsc};
     pf_launch(1, pf_route_kernel, dim3((nt + 3) / 4), dim3(512), 0, s, RA);
     if ((rc = hipGetLastError())) return rc;
-    pf_launch(10, pf_count_kernel, dim3(nch), dim3(512), 0, s, counts, (int *)nullptr, (const int *)ids, (const int *)flag, nt);
-    if ((rc = hipGetLastError())) return rc;
-    pf_launch(2, pf_scan_kernel, dim3(1), dim3(512), 0, s, counts, nch, offsets, tt, sh ? nt : 0, (const int *)nullptr,
-              (int *)nullptr);
-    if ((rc = hipGetLastError())) return rc;
-    pf_launch(3, pf_fill_kernel, dim3(nch), dim3(512), 0, s, row_token, row_slot, (const int *)counts, (const int *)ids,
-              (const int *)flag, nt, row_sx, (const float *)xsc);
-    if ((rc = hipGetLastError())) return rc;
+    if (nt <= PD_MAX) {
+        pf_launch(2, pf_dispatch_kernel, dim3(1), dim3(512), 0, s, offsets, tt, sh ? nt : 0, row_token, row_slot,
+                  (const int *)ids, (const int *)flag, nt, row_sx, (const float *)xsc);
+        if ((rc = hipGetLastError())) return rc;
+    } else {
+        pf_launch(10, pf_count_kernel, dim3(nch), dim3(512), 0, s, counts, (int *)nullptr, (const int *)ids, (const int *)flag, nt);
+        if ((rc = hipGetLastError())) return rc;
+        pf_launch(2, pf_scan_kernel, dim3(1), dim3(512), 0, s, counts, nch, offsets, tt, sh ? nt : 0, (const int *)nullptr,
+                  (int *)nullptr);
+        if ((rc = hipGetLastError())) return rc;
+        pf_launch(3, pf_fill_kernel, dim3(nch), dim3(512), 0, s, row_token, row_slot, (const int *)counts, (const int *)ids,
+                  (const int *)flag, nt, row_sx, (const float *)xsc);
+        if ((rc = hipGetLastError())) return rc;
+    }
     // grouped GEMMs: one launch over every group (dense experts, the shared
     // expert, the others); qg_prefill_int8_dense splits the dense experts off
     const int grid = qg_cu_count();

@@ -53,7 +53,27 @@ def test_sparse_short_groups(layer, nt):
     P.check_outputs(fw, L, H, x, P.sample_rows(nt, 8, nt), f"short groups D={L.spec.width} nt={nt}")
 
 
-@pytest.mark.parametrize("limit", [448, 640, 768, 896, 1280])
+@pytest.mark.parametrize("nt", [1, 2, 4, 17])
+@pytest.mark.parametrize("name", ["1024-iq4", "1024-q4k"])
+def test_sparse_decode_widths(qgl, name, nt):
+    """Decode batches of a width without decode kernels, direct and residual
+    form: routing, outputs, and the workspace of the batch's own size."""
+    from nebula_amd import qg
+    spec = synth.LayerSpec(**LAYERS[name])
+    L, H = synth.build_layer(spec), P.host_layer(spec)
+    x = synth.inputs(550 + nt, nt, spec.width, correlated=True)
+    fw = P.forward(L, x)
+    P.check_routing(fw, H, x)
+    P.check_outputs(fw, L, H, x, np.arange(nt), f"{name} nt={nt}")
+    h = qg.Device(x)
+    xn, out = qg.Device(np.zeros_like(x)), qg.Device(np.zeros_like(x))
+    qg.call("moe_forward_residual", h.p, fw.ids.p, fw.w.p, fw.flags.p, None, xn.p, out.p, nt, qg.C.byref(L.desc), fw.ws.p, fw.ws_bytes)
+    qg.call("sync")
+    np.testing.assert_array_equal(h.get().view('u4'), (x + out.get()).view('u4'))
+    P.assert_close(out.get(), H.forward(xn.get(), fetch=P.fetcher(L))[0], "residual form")
+
+
+@pytest.mark.parametrize("limit", [256, 448, 640, 768, 896, 1280])
 def test_sparse_limits_agree(layer, limit):
     """A batch at a limit and one token above it: the shared rows agree (the
     kernels differ in the order of their fp32 sums only)."""
