@@ -74,8 +74,16 @@ __global__ __launch_bounds__(512, OCC) void xm_kernel(XmArgs A) {
     constexpr int TOK = S::TOK, ROWS = S::ROWS, RB = S::RB, TF = S::TF;
     constexpr int NX = (TOK + 15) / 16, NW = RB ? 0 : RR;   // 16-byte copies per wave and chunk
     extern __shared__ uint4 s_dyn[];
+    constexpr bool LUT = TYPE == QT_IQ4_NL && N16 >= 2;
+    __shared__ float s_lut[LUT ? 16 : 1];
+    if (LUT && threadIdx.x < 16) s_lut[threadIdx.x] = (float)qg_iq4nl_lut[threadIdx.x];
     uint8_t *lds = (uint8_t *)s_dyn;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    // two wide workgroups share a CU and would run their operand reads and
+    // their products in step; a standing difference in priority lets one's
+    // products run under the other's reads (z 6144 x 2560, 2048 tokens: 731 ->
+    // 720 us)
+    if (N16 >= 2 && ((blockIdx.x >> 8) & 1)) __builtin_amdgcn_s_setprio(1);
     int tt, rt;
     xm_tile(blockIdx.x, A.ntt, A.nrt, tt, rt);
     const int t0 = tt * TOK, r0 = rt * ROWS, n = min(TOK, A.nt - t0), nr = min(ROWS, A.rows - r0);
@@ -177,13 +185,21 @@ __global__ __launch_bounds__(512, OCC) void xm_kernel(XmArgs A) {
                 } else {
                     // chains below 16 are the low nibbles of a block's bytes
                     const uint8_t *k = p + 72 * h + 2 + (chain & 15);
-                    uint32_t q = k[0] | ((uint32_t)k[18] << 8) | ((uint32_t)k[36] << 16) | ((uint32_t)k[54] << 24);
-                    q = iq4_lookup((q >> (4 * (lane >> 5))) & 0x0F0F0F0Fu);  // table value + 128 per byte
+                    const uint32_t sh = 4 * (lane >> 5);
                     const float4 d = *(const float4 *)(tb + r * (16 * TF) + 4 * h);
-                    b[0][r] = d.x * ((float)(q & 0xffu) - 128.0f);
-                    b[1][r] = d.y * ((float)((q >> 8) & 0xffu) - 128.0f);
-                    b[2][r] = d.z * ((float)((q >> 16) & 0xffu) - 128.0f);
-                    b[3][r] = d.w * ((float)(q >> 24) - 128.0f);
+                    if constexpr (N16 >= 2) {  // fewer vector instructions (6144 x 2560, 2048 tokens: 832 -> 799 us)
+                        b[0][r] = d.x * s_lut[(k[0] >> sh) & 15];
+                        b[1][r] = d.y * s_lut[(k[18] >> sh) & 15];
+                        b[2][r] = d.z * s_lut[(k[36] >> sh) & 15];
+                        b[3][r] = d.w * s_lut[(k[54] >> sh) & 15];
+                    } else {                   // no second trip to shared memory
+                        uint32_t q = k[0] | ((uint32_t)k[18] << 8) | ((uint32_t)k[36] << 16) | ((uint32_t)k[54] << 24);
+                        q = iq4_lookup((q >> sh) & 0x0F0F0F0Fu);  // table value + 128 per byte
+                        b[0][r] = d.x * ((float)(q & 0xffu) - 128.0f);
+                        b[1][r] = d.y * ((float)((q >> 8) & 0xffu) - 128.0f);
+                        b[2][r] = d.z * ((float)((q >> 16) & 0xffu) - 128.0f);
+                        b[3][r] = d.w * ((float)(q >> 24) - 128.0f);
+                    }
                 }
             }
         }
@@ -242,6 +258,10 @@ __global__ __launch_bounds__(512, OCC) void xm_kernel(XmArgs A) {
                 }
             }
             weights(c * CH + q, b);
+            // a small IQ4_NL tile's operands are ready before the first product
+            // (17 tokens, 2560 x 6144: 27.2 -> 25.3 us; Q4_K, Q8_0 and the wide
+            // tiles lose by it)
+            if (TYPE == QT_IQ4_NL && N16 < 2) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
 #pragma unroll
