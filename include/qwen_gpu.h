@@ -195,7 +195,7 @@ void qg_host_free(void *p);
  * Prefill: 0 router, 1 routing, 2 scan, 3 fill, 4 gate/up dense pass,
  * 5 gate/up other experts, 6 down dense pass, 7 down other experts,
  * 8 shared-expert down (when its format differs), 9 combine, 10 chunk
- * histogram.  n <= 32;
+ * histogram (up to 256 tokens 2 covers 3 and 10 too).  n <= 32;
  * n = 0 disables. */
 int qg_moe_kernel_events(void **events, int n);
 

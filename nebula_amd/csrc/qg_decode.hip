@@ -758,11 +758,11 @@ QG_DEV void gu3_selections(const GuArgs &A, const int *ids, int e, int M, const 
 
 // The workgroup's blocks rb0 .. rb1 - 1 of one expert with M tiles, whose
 // first GU3_RING - 1 blocks' copies are in flight; tn / tt: the tiles' token
-// counts and tokens, tq: their selections (written by wave 0 here, read after
-// the first block's barrier), all in shared memory.
+// counts and tokens, tq: their selections (with sel written by wave 0 here, read
+// after the first block's barrier), all in shared memory.
 template <int M>
 QG_DEV void gu3_run(const GuArgs &A, const int *ids, int e, int rb0, int rb1, const int *tn, const int (*tt)[TILE_TOK],
-                    int (*tq)[TILE_TOK], int k0, uint4 *s_dyn, int tid) {
+                    int (*tq)[TILE_TOK], int k0, uint4 *s_dyn, int tid, bool sel) {
     const int wave = tid >> 6, lane = tid & 63, j = lane & 15, kq = lane >> 4;
     const int D = A.D, D32 = D / 32, nb = rb1 - rb0;
     const uint8_t *gm = e < 0 ? A.sh_gate : A.gate + (size_t)e * A.F * A.rb;
@@ -784,7 +784,7 @@ QG_DEV void gu3_run(const GuArgs &A, const int *ids, int e, int rb0, int rb1, co
         for (int f = 0; f < 8; f++) af[m][f] = real ? ld_frag(xr + f * 32) : qg_half8{};
         sf[m] = (kq || !real) ? qg_half8{} : ld_frag(xs);
     }
-    if (wave == 0) gu3_selections(A, ids, e, M, tn, tt, tq, k0, lane);
+    if (sel && wave == 0) gu3_selections(A, ids, e, M, tn, tt, tq, k0, lane);
     auto copy_block = [&](int rb, int s) { gu3_copy(A, gm, um, rb, ring + (size_t)s * GU3_SLOT, wave, lane); };
     const int fmt = e < 0 ? A.sh_fmt : A.fmt;
     for (int it = 0; it < nb; it++) {
@@ -844,6 +844,7 @@ QG_DEV void gu3_run(const GuArgs &A, const int *ids, int e, int rb0, int rb1, co
 // chose it (the routing kernel's per-expert masks), cut into tiles of up to 8
 // tokens in token order; the routed tiles are numbered in list order and
 // published by each expert's first workgroup for the down kernel.
+template <bool SPAN>
 __global__ __launch_bounds__(512, 1) void dec_gateup3_kernel(GuArgs A) {
     extern __shared__ uint4 s_dyn[];
     // the expert list, in the second partial-sum buffer (first written after
@@ -853,7 +854,8 @@ __global__ __launch_bounds__(512, 1) void dec_gateup3_kernel(GuArgs A) {
     uint32_t *s_xt = (uint32_t *)(s_cum + GU3_MAXX + 1);
     int *s_ids = (int *)(s_xt + GU3_MAXX);  // the routing ids, so the selections need no global reads behind the copies
     __shared__ int s_nx;
-    __shared__ int s_tq[GU3_MAXT][TILE_TOK], s_tt[GU3_MAXT][TILE_TOK], s_tn[GU3_MAXT];
+    // tiles of the workgroup's piece of one expert (or two pieces, see below)
+    __shared__ int s_tq[2][GU3_MAXT][TILE_TOK], s_tt[2][GU3_MAXT][TILE_TOK], s_tn[2][GU3_MAXT];
     const uint32_t G = entry_grid();
     entry_args(A);
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -952,10 +954,95 @@ __global__ __launch_bounds__(512, 1) void dec_gateup3_kernel(GuArgs A) {
     __syncthreads();
     const int nx = s_nx;
     if (nx == 0) return;  // block-uniform: nothing computed on the device
+    const uint32_t C = (uint32_t)s_cum[nx], g = blockIdx.x;
+    // the tiles of list entry xx (n tokens each, in token order) as piece p, by one wave
+    auto list_tiles = [&](int xx, int p) {
+        const int m = lane >> 3, slot = lane & 7;
+        if (m >= s_xm[xx]) return;
+        int n, t = 0;
+        if (s_xe[xx] < 0) {
+            n = min(TILE_TOK, A.nt - TILE_TOK * m);
+            t = TILE_TOK * m + slot;
+        } else {
+            const uint32_t msk = s_xt[xx];
+            n = min(TILE_TOK, __popc(msk) - TILE_TOK * m);
+            // the (8 m + slot)-th set bit of the mask, found by halving
+            int k = TILE_TOK * m + slot;
+#pragma unroll
+            for (int w = 16; w >= 1; w >>= 1) {
+                const int c = __popc((msk >> t) & ((1u << w) - 1u));
+                if (k >= c) { k -= c; t += w; }
+            }
+        }
+        if (slot < n) s_tt[p][m][slot] = t;
+        if (slot == 0) s_tn[p][m] = n;
+    };
+    auto first_copies = [&](int e, int rb0, int rb1) {
+        const uint8_t *gm = e < 0 ? A.sh_gate : A.gate + (size_t)e * A.F * A.rb;
+        const uint8_t *um = e < 0 ? A.sh_up : A.up + (size_t)e * A.F * A.rb;
+        uint4 *ring = s_dyn + (size_t)wave * GU3_RING * GU3_SLOT;
+        for (int i = 0; i < GU3_RING - 1 && rb0 + i < rb1; i++) gu3_copy(A, gm, um, rb0 + i, ring + (size_t)i * GU3_SLOT, wave, lane);
+    };
+    auto run = [&](int M, int e, int rb0, int rb1, int p, int k0, bool sel) {
+        if (M == 1) gu3_run<1>(A, s_ids, e, rb0, rb1, s_tn[p], s_tt[p], s_tq[p], k0, s_dyn, tid, sel);
+        else if (M == 2) gu3_run<2>(A, s_ids, e, rb0, rb1, s_tn[p], s_tt[p], s_tq[p], k0, s_dyn, tid, sel);
+        else gu3_run<3>(A, s_ids, e, rb0, rb1, s_tn[p], s_tt[p], s_tq[p], k0, s_dyn, tid, sel);
+    };
+    if constexpr (SPAN) {
+        // Whole workgroups per expert leave shares that differ up to twofold
+        // when there are few per expert (147 experts on 256 workgroups: one or
+        // two each).  Then a share is an equal part of the cost line, which may
+        // end one expert and begin the next (an expert costs at least
+        // (GU3_COST + 1) RBK, so two at most); the second piece costs about
+        // three blocks of latency.  Taken where this estimate says so: 17
+        // independent tokens 97.3 -> 81.1 us a layer, 14 79.7 -> 72.7, 10 64.9 ->
+        // 61.9.
+        const uint32_t one = (GU3_COST + 1) * (uint32_t)RBK;   // a one-tile expert's cost
+        const float wgs = fmaxf(1.0f, floorf((float)(G * one) * __builtin_amdgcn_rcpf((float)C)));  // its workgroups
+        if (C <= one * G && (float)(one * G) * __builtin_amdgcn_rcpf(wgs) > (float)(C + 3 * (GU3_COST + 1) * G)) {
+            const uint32_t lo = (uint32_t)((unsigned long long)C * g / G), hi = (uint32_t)((unsigned long long)C * (g + 1) / G);
+            int x = 0;
+            for (int c0 = 0; c0 < nx; c0 += 64) {
+                const int xx = c0 + lane;
+                x += __popcll(__ballot(xx < nx && (uint32_t)s_cum[xx + 1] <= lo));
+            }
+            int pe[2], pM[2], p0[2], p1[2];
+#pragma unroll
+            for (int p = 0; p < 2; p++) {
+                const int xx = min(x + p, nx - 1);
+                const uint32_t cum = (uint32_t)s_cum[xx], end = (uint32_t)s_cum[xx + 1];
+                pe[p] = s_xe[xx];
+                pM[p] = s_xm[xx];
+                const uint32_t cpb = (uint32_t)(GU3_COST + pM[p]);
+                const bool any = x + p < nx && cum < hi;
+                p0[p] = lo > cum ? (int)((lo - cum + cpb - 1) / cpb) : 0;
+                p1[p] = !any ? 0 : hi >= end ? RBK : (int)((hi - cum + cpb - 1) / cpb);
+            }
+            const int f = p0[0] < p1[0] ? 0 : 1;   // the first piece may be empty
+            if (p0[f] < p1[f]) first_copies(pe[f], p0[f], p1[f]);
+            // both pieces' tiles and selections before the first run, which
+            // overwrites the list
+            if (wave < 2 && p0[wave] < p1[wave]) {
+                const int xx = min(x + wave, nx - 1), k0 = p0[wave] == 0 && s_xe[xx] >= 0 ? s_xk[xx] : -1;
+                list_tiles(xx, wave);
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                gu3_selections(A, s_ids, s_xe[xx], s_xm[xx], s_tn[wave], s_tt[wave], s_tq[wave], k0, lane);
+            }
+            __syncthreads();
+            if (p0[f] < p1[f]) run(pM[f], pe[f], p0[f], p1[f], f, -1, false);
+            if (f == 0 && p0[1] < p1[1]) {  // block-uniform
+                __syncthreads();  // the first piece's last sums have been read
+                first_copies(pe[1], p0[1], p1[1]);
+                run(pM[1], pe[1], p0[1], p1[1], 1, -1, false);
+            }
+            return;
+        }
+    }
     // this workgroup's expert: the one whose cost range holds the midpoint of
     // its share; its blocks are split evenly over the expert's workgroups
     // (C <= RBK (GU3_COST + 3) 173 and G <= 1024: 32-bit products suffice)
-    const uint32_t C = (uint32_t)s_cum[nx], g = blockIdx.x;
     const uint32_t pos = ((2 * g + 1) * C) / (2 * G);
     int x = 0;
     for (int c0 = 0; c0 < nx; c0 += 64) {
@@ -971,44 +1058,14 @@ __global__ __launch_bounds__(512, 1) void dec_gateup3_kernel(GuArgs A) {
     const uint32_t gA = first_wg(x), gB = first_wg(x + 1), W = gB - gA, kx = g - gA;
     const int rb0 = (int)(RBK * kx / W), rb1 = (int)(RBK * (kx + 1) / W);
     const int e = s_xe[x], M = s_xm[x], k0 = kx == 0 && e >= 0 ? s_xk[x] : -1;
-    // the first blocks' weights go out first
-    {
-        const uint8_t *gm = e < 0 ? A.sh_gate : A.gate + (size_t)e * A.F * A.rb;
-        const uint8_t *um = e < 0 ? A.sh_up : A.up + (size_t)e * A.F * A.rb;
-        uint4 *ring = s_dyn + (size_t)wave * GU3_RING * GU3_SLOT;
-        for (int i = 0; i < GU3_RING - 1 && rb0 + i < rb1; i++) gu3_copy(A, gm, um, rb0 + i, ring + (size_t)i * GU3_SLOT, wave, lane);
-    }
-    if (wave == 0) {
-        // the expert's tiles: n tokens each, in token order
-        const int m = lane >> 3, slot = lane & 7;
-        if (m < M) {
-            int n, t = 0;
-            if (e < 0) {
-                n = min(TILE_TOK, A.nt - TILE_TOK * m);
-                t = TILE_TOK * m + slot;
-            } else {
-                const uint32_t msk = s_xt[x];
-                n = min(TILE_TOK, __popc(msk) - TILE_TOK * m);
-                // the (8 m + slot)-th set bit of the mask, found by halving
-                int k = TILE_TOK * m + slot;
-#pragma unroll
-                for (int w = 16; w >= 1; w >>= 1) {
-                    const int c = __popc((msk >> t) & ((1u << w) - 1u));
-                    if (k >= c) { k -= c; t += w; }
-                }
-            }
-            if (slot < n) s_tt[m][slot] = t;
-            if (slot == 0) s_tn[m] = n;
-        }
-    }
+    first_copies(e, rb0, rb1);  // the first blocks' weights go out first
+    if (wave == 0) list_tiles(x, 0);
     __syncthreads();
     if (rb1 <= rb0) {  // block-uniform: no blocks here; the first workgroup still publishes
-        if (wave == 0 && k0 >= 0) gu3_selections(A, s_ids, e, M, s_tn, s_tt, s_tq, k0, lane);
+        if (wave == 0 && k0 >= 0) gu3_selections(A, s_ids, e, M, s_tn[0], s_tt[0], s_tq[0], k0, lane);
         return;
     }
-    if (M == 1) gu3_run<1>(A, s_ids, e, rb0, rb1, s_tn, s_tt, s_tq, k0, s_dyn, tid);
-    else if (M == 2) gu3_run<2>(A, s_ids, e, rb0, rb1, s_tn, s_tt, s_tq, k0, s_dyn, tid);
-    else gu3_run<3>(A, s_ids, e, rb0, rb1, s_tn, s_tt, s_tq, k0, s_dyn, tid);
+    run(M, e, rb0, rb1, 0, k0, true);
 }
 
 // Shared-memory layout of the gate/up kernel (fp16 units): 16 staged plane
@@ -1753,7 +1810,11 @@ int dec_forward(float *out, float *resid, int *ids, float *weights, unsigned cha
         // workgroup per CU, each on one expert's run of F blocks
         // (one token: the per-tile kernel with its finer split, 512 workgroups)
         if (inl) dec_launch(2, dec_gateup2_kernel<true>, dim3(nwg2), dim3(256), GU2_LDS, s, G2);
-        else dec_launch(2, dec_gateup3_kernel, dim3(qg_cu_count()), dim3(64 * GU3_W), GU3_LDS, s, G2);
+        // batches of 9 and more may touch so many experts that shares must span
+        // two of them; below, whole workgroups per expert are the better split (8
+        // independent tokens: 52.3 us a layer, 53.7 spanning)
+        else if (nt > GU3_W) dec_launch(2, dec_gateup3_kernel<true>, dim3(qg_cu_count()), dim3(64 * GU3_W), GU3_LDS, s, G2);
+        else dec_launch(2, dec_gateup3_kernel<false>, dim3(qg_cu_count()), dim3(64 * GU3_W), GU3_LDS, s, G2);
     } else {
         // D = 2560 (dec_ok): the register-weight kernel, 10 superblocks per row
         const size_t gu_bytes = (size_t)gu_lds(D).total * 2;

@@ -73,6 +73,21 @@ def test_sparse_decode_widths(qgl, name, nt):
     P.assert_close(out.get(), H.forward(xn.get(), fetch=P.fetcher(L))[0], "residual form")
 
 
+@pytest.mark.parametrize("nt", [9, 10, 14, 17])
+@pytest.mark.parametrize("name", ["2048-iq4", "2048-q4k"])
+def test_decode_shares_span_experts(qgl, name, nt):
+    """Verify batches of independent tokens touch so many experts that a
+    gate/up workgroup's share may end one and begin the next; a second call
+    with one context's tokens goes back to whole workgroups per expert."""
+    spec = synth.LayerSpec(**LAYERS[name])
+    L, H = synth.build_layer(spec), P.host_layer(spec)
+    for corr in (False, True):
+        x = synth.inputs(560 + nt, nt, spec.width, correlated=corr)
+        fw = P.forward(L, x)
+        P.check_routing(fw, H, x)
+        P.check_outputs(fw, L, H, x, np.arange(nt), f"{name} nt={nt} corr={corr}")
+
+
 @pytest.mark.parametrize("limit", [256, 448, 640, 768, 896, 1280])
 def test_sparse_limits_agree(layer, limit):
     """A batch at a limit and one token above it: the shared rows agree (the
