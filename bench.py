@@ -572,7 +572,7 @@ def bench_matmul(args, data) -> dict:
             "vs_baseline": None, "dtype": "f32", "data": data,
             "config": {"workload": f"qg_matmul, Q4_K, D=2560 dense projections (qkv 10240x2560, z 6144x2560, out 2560x6144), "
                                    f"{nt} tokens, exact reference order", "batch_tokens": nt, "per_shape": per},
-            "roofline": {"bound": "hbm", "kernel": "mm_tile_kernel (qkv)", "achieved": achieved, "peak": 8000.0, "unit": "GB/s",
+            "roofline": {"bound": "hbm", "kernel": f"{'mm_tile_kernel' if nt <= 4 else 'xm_kernel'} (qkv)", "achieved": achieved, "peak": 8000.0, "unit": "GB/s",
                          "frac": round(achieved / 8000.0, 4), "traffic": None},
             "cpu_baseline": cpu}
 
