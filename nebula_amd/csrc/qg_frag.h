@@ -94,13 +94,47 @@ QG_DEV qg_half8 gq_frag(uint4 c, int f, _Float16 sc, _Float16 of) {
     return r;
 }
 QG_DEV qg_half8 ld_frag(const _Float16 *p) { return __builtin_bit_cast(qg_half8, *(const uint4 *)p); }
+// The min term of one Q4_K superblock, sum_g m_g X_g over its eight groups, for
+// the 16 plane rows of a fragment.  Two forms of the group sums X_g:
+// MinPlanes: two fp16 values each ([row][2][K / 32]), one fp16 product.
+struct MinPlanes {
+    typedef qg_half8 Sums;
+    qg_half8 b;
+    __device__ __forceinline__ MinPlanes(const Q4kHeader &h, int) : b(q4k_min_frag(h)) {}
+    __device__ __forceinline__ qg_f4 term(const Sums &s) const {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(s, b, qg_f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+    }
+    // superblock sb's sums of row `row` (nsb superblocks per row) as lane (j, kq) feeds them
+    static __device__ __forceinline__ Sums load(const _Float16 *sums, size_t row, int nsb, int sb, int j, int kq) {
+        const qg_half8 v = ld_frag(sums + ((row * 2 + (j & 1)) * nsb + sb) * 8);
+        return kq ? qg_half8{} : v;
+    }
+};
+// MinF32: fp32 ([row][K / 32], the same bytes), two fp32 products of four
+// groups; the hi plane's rows carry the sums, the lo plane's zeros.
+struct MinF32 {
+    typedef float2 Sums;
+    float b0, b1;
+    __device__ __forceinline__ MinF32(const Q4kHeader &h, int kq)
+        : b0((float)((h.M[0] >> (8 * kq)) & 0xffu)), b1((float)((h.M[1] >> (8 * kq)) & 0xffu)) {}
+    __device__ __forceinline__ qg_f4 term(const Sums &s) const {
+        const qg_f4 t = __builtin_amdgcn_mfma_f32_16x16x4f32(s.x, b0, qg_f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(s.y, b1, t, 0, 0, 0);
+    }
+    static __device__ __forceinline__ Sums load(const _Float16 *sums, size_t row, int nsb, int sb, int j, int kq) {
+        const float *p = (const float *)sums + (row * nsb + sb) * 8 + kq;
+        const float2 v = make_float2(p[0], p[4]);
+        return (j & 1) ? make_float2(0.0f, 0.0f) : v;
+    }
+};
+
 // A wave's products of one superblock of 16 gate and 16 up Q4_K rows (9 pieces
 // of 16 bytes each at wb, rotated by row / 8) with M tiles of 8 token rows
-// (af: their hi and lo planes as the 16 rows of a fragment, sf: the planes of
-// the group sums): y[cb][m] = the partial sums for the 16 gate (cb 0) or up (cb 1) rows, column j,
+// (af: their hi and lo planes as the 16 rows of a fragment, sf: their group
+// sums): y[cb][m] = the partial sums for the 16 gate (cb 0) or up (cb 1) rows, column j,
 // as (token 2kq, token 2kq + 1) with the hi and lo plane rows added.
-template <int M, int MT>
-QG_DEV void ksplit_products(const uint4 *wb, const qg_half8 (&af)[MT][8], const qg_half8 (&sf)[MT], int j, int kq,
+template <int M, typename MIN = MinPlanes, int MT>
+QG_DEV void ksplit_products(const uint4 *wb, const qg_half8 (&af)[MT][8], const typename MIN::Sums (&sf)[MT], int j, int kq,
                             float2 (&y)[2][MT]) {
     static_assert(M <= MT, "tiles");
 #pragma unroll
@@ -113,9 +147,9 @@ QG_DEV void ksplit_products(const uint4 *wb, const qg_half8 (&af)[MT][8], const 
         qg_half2 scA, ofA, scB, ofB;  // scales of groups gA, gA + 1 and gB, gB + 1
         gq_scales(h.S[0], kq, scA, ofA);
         gq_scales(h.S[1], kq, scB, ofB);
-        qg_f4 p0[M], p1[M], mm[M];
+        qg_f4 p0[M], p1[M];
 #pragma unroll
-        for (int m = 0; m < M; m++) p0[m] = p1[m] = mm[m] = qg_f4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int m = 0; m < M; m++) p0[m] = p1[m] = qg_f4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int f = 0; f < 4; f++) {
             const qg_half8 b0 = gq_frag(ch0, f, scA[f >> 1], ofA[f >> 1]), b1 = gq_frag(ch1, f, scB[f >> 1], ofB[f >> 1]);
@@ -125,13 +159,13 @@ QG_DEV void ksplit_products(const uint4 *wb, const qg_half8 (&af)[MT][8], const 
                 p1[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[m][4 + f], b1, p1[m], 0, 0, 0);
             }
         }
-        const qg_half8 bm = q4k_min_frag(h);
+        const MIN mins(h, kq);
 #pragma unroll
         for (int m = 0; m < M; m++) {
-            mm[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(sf[m], bm, mm[m], 0, 0, 0);
+            const qg_f4 mm = mins.term(sf[m]);
             float v[4];
 #pragma unroll
-            for (int i = 0; i < 4; i++) v[i] = __builtin_fmaf(h.d, p0[m][i] + p1[m][i], -h.dmin * mm[m][i]);
+            for (int i = 0; i < 4; i++) v[i] = __builtin_fmaf(h.d, p0[m][i] + p1[m][i], -h.dmin * mm[i]);
             y[cb][m] = make_float2(v[0] + v[1], v[2] + v[3]);
         }
     }
@@ -232,13 +266,13 @@ QG_DEV float lds_rms_scale(const float *xl, int D, float eps, int lane) {
     return 1.0f / __builtin_sqrtf(ss / (float)D + eps);
 }
 
-// The fp16 hi/lo planes of one token row (Q4_K fragment order) and the hi/lo
-// planes of its 32-group sums, optionally RMS-scaled by sc (written to xn);
-// lane g handles groups g, g+64, ... with 8 float4 loads each.  In the Q4_K
+// The fp16 hi/lo planes of one token row (Q4_K fragment order) and its 32-group
+// sums (their hi/lo planes, or in fp32 to `sums`), optionally RMS-scaled by sc
+// (written to xn); lane g handles groups g, g+64, ... with 8 float4 loads each.  In the Q4_K
 // order every 16-byte chunk holds 8 consecutive elements of one group (in
 // qg_perm8 order), so each group is written as 4 chunks per plane.
 QG_DEV void token_planes(const float *xr, int D, bool norm, float sc, int lane, _Float16 *hi, _Float16 *lo,
-                         _Float16 *shi, _Float16 *slo, float *xn) {
+                         _Float16 *shi, _Float16 *slo, float *xn, float *sums = nullptr) {
     for (int g = lane; g < D / 32; g += 64) {
         float v[32];
         const float4 *src = (const float4 *)(xr + 32 * g);
@@ -253,9 +287,13 @@ QG_DEV void token_planes(const float *xr, int D, bool norm, float sc, int lane, 
             if (norm) v[l] = v[l] * sc;
             s += v[l];
         }
-        const _Float16 sh = (_Float16)s;
-        shi[g] = sh;
-        slo[g] = (_Float16)(s - (float)sh);
+        if (sums) {
+            sums[g] = s;
+        } else {
+            const _Float16 sh = (_Float16)s;
+            shi[g] = sh;
+            slo[g] = (_Float16)(s - (float)sh);
+        }
         if (norm && xn) {
             float4 *dst = (float4 *)(xn + 32 * g);
 #pragma unroll

@@ -149,6 +149,7 @@ struct RouteArgs {
     const uint8_t *resident; double thr;
     int *ids; float *w; uint8_t *flags_out; int *flag; int *missing; double *mass;
     const float *x; int D; _Float16 *xp, *xsp;
+    bool sums32;                      // xsp holds the 32-group sums as fp32 [nt][D/32] (decode batches)
     const float *sh_row; float *sh_logit;   // shared gate vector and its logits (sh_logit[t * ld]), or null
     int8_t *xi8; float *xsc;          // int8 planes and row scales (the int8 dense pass), or null
 };
@@ -189,7 +190,8 @@ __global__ __launch_bounds__(512) void pf_route_kernel(RouteArgs A) {
     if (t >= A.nt) return;  // whole wave; no block barrier in this kernel
     if (wave >= 4) {  // the token's activation planes, beside its routing
         _Float16 *hi = A.xp + (size_t)t * 2 * A.D, *shi = A.xsp + (size_t)t * 2 * (A.D / 32);
-        token_planes(A.x + (size_t)t * A.D, A.D, false, 1.0f, lane, hi, hi + A.D, shi, shi + A.D / 32, nullptr);
+        token_planes(A.x + (size_t)t * A.D, A.D, false, 1.0f, lane, hi, hi + A.D, shi, shi + A.D / 32, nullptr,
+                     A.sums32 ? (float *)shi : nullptr);
         if (A.sh_row) {
             const float *xr = A.x + (size_t)t * A.D + (lane & 31), *gr = A.sh_row + (lane & 31);
             float a = 0.0f;
@@ -1398,11 +1400,13 @@ __global__ __launch_bounds__(512, 1) void pf_down_kernel(DnArgs A) {
 //               F 256: 100 tokens 35 / 28, 600 45 / 41, 1500 59 / 76
 // Runs of two tiles hold the mid fragments of K = 512 in registers for Q4_K; the
 // IQ4_NL conversion needs the registers, so it takes one tile there (with two,
-// spills in the loop made 400 tokens 262 us).
+// spills in the loop made 400 tokens 262 us).  Decode batches (qg_prefill_small_ok)
+// take the FULL forms.
 bool pf_gateup_sp(const SpGuArgs &A, int cus, hipStream_t s) {
-    if (A.D == 2048 && A.nt <= 1280) pf_launch(5, pf_gateup_sp_kernel<8, 3>, dim3(cus), dim3(512), SpGu<8, 3>::LDS, s, A);
-    else if (A.D == 2560 && A.nt <= 640) pf_launch(5, pf_gateup_sp_kernel<10, 2>, dim3(cus), dim3(640), SpGu<10, 2>::LDS, s, A);
-    else if (A.D == 1024 && A.nt <= 896) pf_launch(5, pf_gateup_sp_kernel<4, 2>, dim3(2 * cus), dim3(256), SpGu<4, 2>::LDS, s, A);
+    if (A.D == 1024 && A.nt <= QG_MAX_DECODE) pf_launch(5, pf_gateup_sp_kernel<4, 2, true>, dim3(2 * cus), dim3(256), SpGu<4, 2>::LDS, s, A);
+    else if (A.D == 2048 && A.nt <= 1280) pf_launch(5, pf_gateup_sp_kernel<8, 3, false>, dim3(cus), dim3(512), SpGu<8, 3>::LDS, s, A);
+    else if (A.D == 2560 && A.nt <= 640) pf_launch(5, pf_gateup_sp_kernel<10, 2, false>, dim3(cus), dim3(640), SpGu<10, 2>::LDS, s, A);
+    else if (A.D == 1024 && A.nt <= 896) pf_launch(5, pf_gateup_sp_kernel<4, 2, false>, dim3(2 * cus), dim3(256), SpGu<4, 2>::LDS, s, A);
     else return false;
     return true;
 }
@@ -1410,7 +1414,9 @@ bool pf_down_sp(const SpDnArgs &A, int fmt, int F, int cus, hipStream_t s) {
     auto go = [&](auto FC, auto NC, int most) {
         constexpr int FMT = decltype(FC)::value, NB = decltype(NC)::value, TM = FMT == QT_IQ4_NL && NB >= 16 ? 1 : 2;
         if (A.nt > most) return false;
-        pf_launch(7, pf_down_sp_kernel<FMT, NB, TM>, dim3(cus), dim3(512), SpDn<FMT, NB>::LDS, s, A);
+        constexpr bool SUMS = FMT == QT_Q4_K;   // IQ4_NL has no min term
+        if (A.nt <= QG_MAX_DECODE) pf_launch(7, pf_down_sp_kernel<FMT, NB, TM, SUMS>, dim3(cus), dim3(512), SpDn<FMT, NB>::LDS, s, A);
+        else pf_launch(7, pf_down_sp_kernel<FMT, NB, TM, false>, dim3(cus), dim3(512), SpDn<FMT, NB>::LDS, s, A);
         return true;
     };
     using Q4 = std::integral_constant<int, QT_Q4_K>;
@@ -1536,10 +1542,14 @@ size_t qg_prefill_workspace_bytes(int width, int ff, int tokens) {
 }
 
 // Decode batches at widths the decode kernels lack (2048 and 2560 are theirs),
-// for which both GEMM passes have a kernel of qg_sparse.h: the prefill path is
-// ahead of the generic kernels but for 2 and 3 tokens (1024/256, us per layer,
-// generic / prefill: 1 token 41.4 / 35.2, 2 36.5 / 37.1, 4 39.5 / 37.8, 8 55.8 /
-// 39.4, 17 75.9 / 44.2).
+// for which both GEMM passes have a kernel of qg_sparse.h (FULL form, the
+// generic kernels' arithmetic): the prefill path is ahead of the generic
+// kernels but for 2 and 3 tokens (F = 256, independent tokens, us per layer in a
+// graph, generic / prefill: 1 token 34.3 / 33.7, 4 38.8 / 37.6, 8 63.2 / 44.8, 17
+// 101 / 55; F = 512: 36.3 / 35.5, 55.6 / 46.4, 96 / 56, 144 / 69; F = 640: 37.8 /
+// 36.2, 56.9 / 48.8, 90 / 58, 143 / 77).  With the group sums as two fp16 values
+// and the hardware's exponential it was 1 to 6 % shorter; those lose bits and
+// range that the generic kernels have.
 bool qg_prefill_small_shape(int width, int ff) { return width == 1024 && (ff == 256 || ff == 512 || ff == 640); }
 bool qg_prefill_small_ok(const qg_moe_layer *L, int nt) {
     return (nt == 1 || nt > 3) && qg_prefill_small_shape(L->width, L->ff) && qg_prefill_ok(L) && (!L->sh_gate || L->sh_down_type == L->down_type);
@@ -1574,12 +1584,13 @@ int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsig
     else if (xm_wide(QG_EXPERTS, nt)) pf_router<2, 2, 2, 4>(R, s);
     else pf_router<1, 1, 3, 4>(R, s);
     if ((rc = hipGetLastError())) return rc;
-    const int split = tl_pf_split;
+    const bool dec = nt <= QG_MAX_DECODE;   // a decode batch: group sums in fp32, no dense experts to split off
+    const int split = dec ? 0 : tl_pf_split;
     const bool i8 = split == 1;
     int8_t *xi8 = i8 ? (int8_t *)(ws + lay.xi8) : nullptr;
     float *xsc = i8 ? (float *)(ws + lay.xsc) : nullptr, *row_sx = i8 ? (float *)(ws + lay.row_sx) : nullptr;
     RouteArgs RA{nt, logits, rows, L->resident, L->threshold, ids, weights, flags, flag,
-                 (int *)(ws + lay.missing), (double *)(ws + lay.mass), x, D, xp, xsp,
+                 (int *)(ws + lay.missing), (double *)(ws + lay.mass), x, D, xp, xsp, dec,
                  sh ? L->sh_gate_inp : nullptr, logits + QG_EXPERTS, xi8, xsc};
     pf_launch(1, pf_route_kernel, dim3((nt + 3) / 4), dim3(512), 0, s, RA);
     if ((rc = hipGetLastError())) return rc;

@@ -168,6 +168,14 @@ QG_DEV void sp_pin(qg_half8 &f) {
     asm volatile("" : "+v"(v));
     f = __builtin_bit_cast(qg_half8, v);
 }
+QG_DEV void sp_pin(float2 &f) { asm volatile("" : "+v"(f.x), "+v"(f.y)); }
+
+// FULL (decode batches, which take the place of the generic kernels and keep
+// their arithmetic): the group sums of x and of mid in fp32 and SwiGLU with
+// qg_expf and a division, where prefill has two fp16 values and the hardware's
+// exponential and reciprocal.  The sums of 32 values of one sign then reach
+// past 65504, as the values' own planes do.
+template <bool FULL> using SpMin = std::conditional_t<FULL, MinF32, MinPlanes>;
 
 // ---- gate/up: K split over the waves ----
 // Wave w (of W = D / 256) multiplies superblock w of a sub-unit's 16 gate and 16
@@ -195,11 +203,11 @@ struct SpGuArgs {
     const int *offsets, *row_token;
     const uint8_t *gate, *up, *sh_gate, *sh_up; size_t rb;   // Q4_K rows of D
     const _Float16 *xp, *xsp;
-    _Float16 *midp, *msp;            // [rows][2][F] (down format order), [rows][2][F/32]
+    _Float16 *midp, *msp;            // [rows][2][F] (down format order), [rows][2][F/32] (FULL: fp32 [rows][F/32], as xsp)
     int down_fmt, sh_down_fmt;
 };
 
-template <int W, int TM>
+template <int W, int TM, bool FULL>
 __global__ __launch_bounds__(64 * W, 1) void pf_gateup_sp_kernel(SpGuArgs A) {
     extern __shared__ uint4 s_dyn[];
     __shared__ SpList S;
@@ -208,7 +216,8 @@ __global__ __launch_bounds__(64 * W, 1) void pf_gateup_sp_kernel(SpGuArgs A) {
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, j = lane & 15, kq = lane >> 4;
     for (int i = tid; i <= QG_EXPERTS; i += 64 * W) s_off[i] = A.offsets[i];
     __syncthreads();
-    const int D = A.D, F = A.F, D32 = D / 32, nsr = F / 16;   // sub-units per run
+    using MIN = SpMin<FULL>;
+    const int D = A.D, F = A.F, nsr = F / 16;   // sub-units per run
     sp_build<64 * W, TM>(S, s_dyn, s_off, A.nt, A.sh_gate != nullptr, F / 32, sp_part(), gridDim.x);
     const int nsub = 2 * __builtin_amdgcn_readfirstlane(S.pos[1][3] - S.pos[0][3]);
     if (nsub <= 0) return;  // block-uniform
@@ -263,17 +272,16 @@ __global__ __launch_bounds__(64 * W, 1) void pf_gateup_sp_kernel(SpGuArgs A) {
         // activation fragments of this wave's superblock: plane row r = (row
         // r / 2 of the tile, plane r % 2); rows past the tile's repeat its
         // last (their products are never kept)
-        qg_half8 af[M][8], sf[M];
+        qg_half8 af[M][8];
+        typename MIN::Sums sf[M];
 #pragma unroll
         for (int m = 0; m < M; m++) {
             const int n = min(8, R.n - 8 * m), k = R.base + 8 * m + min(j >> 1, n - 1);
             const int tok = sh ? k : A.row_token[k];
             const _Float16 *xr = A.xp + ((size_t)tok * 2 + (j & 1)) * D + (size_t)wave * 256 + kq * 8;
-            const _Float16 *xs = A.xsp + ((size_t)tok * 2 + (j & 1)) * D32 + (size_t)wave * 8;
 #pragma unroll
             for (int f = 0; f < 8; f++) af[m][f] = ld_frag(xr + f * 32);
-            sf[m] = ld_frag(xs);
-            if (kq) sf[m] = qg_half8{};
+            sf[m] = MIN::load(A.xsp, (size_t)tok, W, wave, j, kq);
         }
 #pragma unroll
         for (int m = 0; m < M; m++) {
@@ -295,7 +303,7 @@ __global__ __launch_bounds__(64 * W, 1) void pf_gateup_sp_kernel(SpGuArgs A) {
                 else if (it + 1 < nsub) wait_vmem_but<SP_CPB>();
                 else wait_vmem();
                 float2 y[2][M];
-                ksplit_products<M>(ring + qc * SP_SLOT, af, sf, j, kq, y);
+                ksplit_products<M, MIN>(ring + qc * SP_SLOT, af, sf, j, kq, y);
                 qc = qc == 2 ? 0 : qc + 1;
 #pragma unroll
                 for (int cb = 0; cb < 2; cb++)
@@ -316,7 +324,7 @@ __global__ __launch_bounds__(64 * W, 1) void pf_gateup_sp_kernel(SpGuArgs A) {
                     u += t2 ? ua.y : ua.x;
                 }
                 const int pos = plane_pos(fmt, (sub + c + b) * 16 + j);
-                const float mv = qg_swiglu_fast(g, u);
+                const float mv = FULL ? qg_swiglu(g, u) : qg_swiglu_fast(g, u);
                 if (idx < R.n) {
                     _Float16 *mp = A.midp + (size_t)row * 2 * F;
                     const _Float16 hv = (_Float16)mv;
@@ -339,7 +347,9 @@ __global__ __launch_bounds__(64 * W, 1) void pf_gateup_sp_kernel(SpGuArgs A) {
                 const int sb = sub + c + b;
                 if (sb & 1) {
                     const float sum = s16 + (NB > 1 ? s_gs[wave >= 2 * M ? wave - 2 * M : 0][kq] : half);
-                    if (j == 0 && idx < R.n) {
+                    if (FULL && j == 0 && idx < R.n) {
+                        ((float *)A.msp)[(size_t)row * (F / 32) + (sb >> 1)] = sum;
+                    } else if (j == 0 && idx < R.n) {
                         _Float16 *gp = A.msp + (size_t)row * 2 * (F / 32) + (sb >> 1);
                         const _Float16 hs = (_Float16)sum;
                         gp[0] = hs;
@@ -385,7 +395,7 @@ struct SpDnArgs {
     float *slots;                    // [rows][D]: slot t*10+k, shared rows at nt*10+t
 };
 
-template <int FMT, int NB, int TM>
+template <int FMT, int NB, int TM, bool FULL>
 __global__ __launch_bounds__(512, 1) void pf_down_sp_kernel(SpDnArgs A) {
     using C = SpDn<FMT, NB>;
     constexpr int F = 32 * NB, RB = C::RB, CP = C::CP;
@@ -442,8 +452,10 @@ __global__ __launch_bounds__(512, 1) void pf_down_sp_kernel(SpDnArgs A) {
     auto run = [&](int cnt, auto MC) {
         constexpr int M = decltype(MC)::value;
         const bool sh = R.e == QG_EXPERTS;
+        using MIN = SpMin<FULL>;
         constexpr int NSB = FMT == QT_Q4_K ? NB / 8 : 1;
-        qg_half8 af[M][NB], sf[M][NSB];
+        qg_half8 af[M][NB];
+        typename MIN::Sums sf[M][NSB];
         int sl[M][2];
 #pragma unroll
         for (int m = 0; m < M; m++) {
@@ -453,12 +465,8 @@ __global__ __launch_bounds__(512, 1) void pf_down_sp_kernel(SpDnArgs A) {
 #pragma unroll
             for (int b = 0; b < NB; b++) af[m][b] = ld_frag(mr + b * 32);
             if constexpr (FMT == QT_Q4_K) {
-                const _Float16 *sr = A.msp + (row * 2 + (j & 1)) * (F / 32);
 #pragma unroll
-                for (int s = 0; s < NSB; s++) {
-                    sf[m][s] = ld_frag(sr + 8 * s);
-                    if (kq) sf[m][s] = qg_half8{};
-                }
+                for (int s = 0; s < NSB; s++) sf[m][s] = MIN::load(A.msp, row, NSB, s, j, kq);
             }
 #pragma unroll
             for (int h = 0; h < 2; h++) {
@@ -522,10 +530,10 @@ __global__ __launch_bounds__(512, 1) void pf_down_sp_kernel(SpDnArgs A) {
                             p1[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[m][8 * s + 4 + f], b1, p1[m], 0, 0, 0);
                         }
                     }
-                    const qg_half8 bm = q4k_min_frag(h);
+                    const MIN mins(h, kq);
 #pragma unroll
                     for (int m = 0; m < M; m++) {
-                        const qg_f4 mm = __builtin_amdgcn_mfma_f32_16x16x32_f16(sf[m][s], bm, qg_f4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                        const qg_f4 mm = mins.term(sf[m][s]);
 #pragma unroll
                         for (int i = 0; i < 4; i++)
                             y[m][i] = __builtin_fmaf(h.d, p0[m][i] + p1[m][i], __builtin_fmaf(-h.dmin, mm[i], y[m][i]));
