@@ -1924,6 +1924,7 @@ size_t qg_moe_workspace_bytes(int width, int ff, int tokens) {
     const size_t extra = 2 * (((size_t)MB * width * 4 + 255) & ~(size_t)255);
     size_t d = dec_layout(width, ff).total;
     if (qg_prefill_small_shape(width, ff)) {
+        // (the generic layout, always of 17 tokens, is the larger today)
         const size_t p = qg_prefill_workspace_bytes(width, ff, tokens);
         d = p > d ? p : d;
     }
@@ -1944,7 +1945,7 @@ int qg_moe_forward(float *out, int *ids, float *weights, unsigned char *flags, q
     if (!out || !ids || !weights || !x || !workspace || ws_bytes < qg_moe_workspace_bytes(L->width, L->ff, nt) ||
         !al16(out) || !al16(x) || !al16(workspace))
         return hipErrorInvalidValue;
-    if (nt > MB || (!dec_ok(L) && qg_prefill_small_ok(L, nt)))
+    if (nt > MB || (!dec_ok(L) && qg_prefill_small_ok(L)))
         return qg_prefill_forward(out, nullptr, ids, weights, flags, stats, x, nullptr, 0, nt, L, workspace);
     if (!dec_ok(L)) return qg_generic_forward(out, ids, weights, flags, stats, x, nt, L, workspace, ws_bytes);
     return dec_forward(out, nullptr, ids, weights, flags, stats, x, nullptr, 0, nt, L, (uint8_t *)workspace);
@@ -1974,7 +1975,7 @@ int qg_moe_forward_residual(float *h, int *ids, float *weights, unsigned char *f
     if (!h || !ids || !weights || !workspace || ws_bytes < qg_moe_workspace_bytes(L->width, L->ff, nt) || !al16(h) ||
         !al16(xn_out) || !al16(out) || !al16(workspace))
         return hipErrorInvalidValue;
-    if (nt > MB || (!dec_ok(L) && qg_prefill_small_ok(L, nt)))
+    if (nt > MB || (!dec_ok(L) && qg_prefill_small_ok(L)))
         return qg_prefill_forward(out, h, ids, weights, flags, stats, h, xn_out, 1, nt, L, workspace);
     if (dec_ok(L)) return dec_forward(out, h, ids, weights, flags, stats, h, xn_out, 1, nt, L, (uint8_t *)workspace);
     // generic form: normalise into the workspace tail, run the layer, add

@@ -32,11 +32,12 @@ extern "C" int qg_generic_forward(float *out, int *ids, float *weights, unsigned
 // `slot` of this thread's calls, if any.
 bool qg_kernel_event_pair(int slot, void **begin, void **end);
 
-// The prefill path (18..8192 tokens) of qg_moe_forward(_residual).
+// The prefill path of qg_moe_forward(_residual): 18..8192 tokens, and the decode
+// batches of qg_prefill_small_ok.
 bool qg_prefill_ok(const qg_moe_layer *L);
 // Decode batches that the prefill path serves (widths without decode kernels).
 bool qg_prefill_small_shape(int width, int ff);
-bool qg_prefill_small_ok(const qg_moe_layer *L, int nt);
+bool qg_prefill_small_ok(const qg_moe_layer *L);
 size_t qg_prefill_workspace_bytes(int width, int ff, int tokens);
 int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsigned char *flags, qg_prune_stats *stats,
                        const float *x, float *xn_out, int norm, int nt, const qg_moe_layer *L, void *workspace);

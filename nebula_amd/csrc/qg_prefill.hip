@@ -1543,16 +1543,17 @@ size_t qg_prefill_workspace_bytes(int width, int ff, int tokens) {
 
 // Decode batches at widths the decode kernels lack (2048 and 2560 are theirs),
 // for which both GEMM passes have a kernel of qg_sparse.h (FULL form, the
-// generic kernels' arithmetic): the prefill path is ahead of the generic
-// kernels but for 2 and 3 tokens (F = 256, independent tokens, us per layer in a
-// graph, generic / prefill: 1 token 34.3 / 33.7, 4 38.8 / 37.6, 8 63.2 / 44.8, 17
-// 101 / 55; F = 512: 36.3 / 35.5, 55.6 / 46.4, 96 / 56, 144 / 69; F = 640: 37.8 /
-// 36.2, 56.9 / 48.8, 90 / 58, 143 / 77).  With the group sums as two fp16 values
-// and the hardware's exponential it was 1 to 6 % shorter; those lose bits and
-// range that the generic kernels have.
+// generic kernels' arithmetic): the prefill path instead of the generic kernels
+// (independent tokens, us per layer in a graph, generic / prefill: F = 256 1 token
+// 34.2 / 34.2, 2 34.1 / 34.8, 4 39.1 / 37.7, 8 63 / 45, 17 101 / 55; F = 512 36.7
+// / 35.5, 39.4 / 37.9, 55.7 / 46.5, 96 / 56, 144 / 69; F = 640 37.8 / 36.3, 40.8 /
+// 39.0, 56.9 / 49.8, 90 / 58, 143 / 77).  All of 1..17 take it, also where the
+// two are level, so that a token's output does not depend on its batch.  With the group
+// sums as two fp16 values and the hardware's exponential it was 1 to 6 % shorter;
+// those lose bits and range that the generic kernels have.
 bool qg_prefill_small_shape(int width, int ff) { return width == 1024 && (ff == 256 || ff == 512 || ff == 640); }
-bool qg_prefill_small_ok(const qg_moe_layer *L, int nt) {
-    return (nt == 1 || nt > 3) && qg_prefill_small_shape(L->width, L->ff) && qg_prefill_ok(L) && (!L->sh_gate || L->sh_down_type == L->down_type);
+bool qg_prefill_small_ok(const qg_moe_layer *L) {
+    return qg_prefill_small_shape(L->width, L->ff) && qg_prefill_ok(L) && (!L->sh_gate || L->sh_down_type == L->down_type);
 }
 
 int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsigned char *flags, qg_prune_stats *stats,

@@ -114,3 +114,14 @@ def test_decode_resident(qgl, name, nt):
     for k in ("token_layers", "missing_selections", "skipped_selections", "avoided_token_handoffs"):
         assert getattr(got, k) == getattr(want_stats, k), k
     assert got.skipped_mass == pytest.approx(want_stats.skipped_mass, rel=1e-12)  # doubles, another order of at most 17
+
+
+@pytest.mark.parametrize("name", ["256-q4k", "640-iq4"])
+def test_decode_batch_independent(qgl, name):
+    """A token's output has the same bits alone and in every decode batch."""
+    L, _ = make(name)
+    x = synth.inputs(630, 17, 1024, correlated=True)
+    whole = P.forward(L, x).out.get()[:17]
+    for nt in (1, 2, 3, 4, 9):
+        got = P.forward(L, x[:nt]).out.get()[:nt]
+        np.testing.assert_array_equal(got.view('u4'), whole[:nt].view('u4'), err_msg=f"{name} nt={nt}")
