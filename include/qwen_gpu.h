@@ -103,9 +103,11 @@ int qg_moe_dispatch(int *offsets, int *row_token, int *row_slot, int *status, co
  * accumulation: each weight enters exactly (Q4_K as the integer s*q, at most
  * 945; IQ4_NL as its table value), each activation as two fp16 planes (hi =
  * fp16(x), lo = fp16(x - hi), about 22 significant bits), superblock and
- * block scales and the Q4_K min term applied in fp32; outputs agree with the
- * reference's fp32 path within max-abs 1e-3 / rel-L2 1e-4 (about 1e-6
- * relative in practice). */
+ * block scales and the Q4_K min term applied in fp32 (the sums of 32 activations
+ * that the min term multiplies are held like activations, as two fp16 values,
+ * whose range is +-65504; in fp32 by the generic kernels and the batches of up
+ * to 17 tokens at D = 1024); outputs agree with the reference's fp32 path
+ * within max-abs 1e-3 / rel-L2 1e-4 (about 1e-6 relative in practice). */
 typedef struct {
     int width, ff;                              /* D, F */
     const float *router;                        /* F32 [512, D] (ffn_gate_inp) */
@@ -136,9 +138,12 @@ size_t qg_moe_workspace_bytes(int width, int ff, int tokens);
  * Device pointers to weights, activations, outputs and the workspace must be
  * 16-byte aligned (qg_alloc returns 256-byte aligned memory); otherwise the
  * call returns an invalid-value error and launches nothing.
- * tokens 1..8192: up to 17 the decode kernels (any format qg_matmul takes);
+ * tokens 1..8192: up to 17 any format qg_matmul takes (the decode kernels, at
+ * D = 1024 the prefill's, or the generic ones; qg_moe_kernel_events lists which);
  * above, the prefill grouped GEMMs, which need Q4_K gate/up, Q4_K or IQ4_NL
- * down, D a multiple of 256 and F a multiple of 128 (else an error). */
+ * down, D a multiple of 256 and F a multiple of 128 (else an error).  The order
+ * of the fp32 sums, and so an output's last bits, may differ between shapes and
+ * batch sizes. */
 int qg_moe_forward(float *out, int *ids, float *weights, unsigned char *flags, qg_prune_stats *stats,
                    const float *x, int tokens, const qg_moe_layer *layer, void *workspace, size_t workspace_bytes);
 
@@ -190,9 +195,11 @@ void qg_host_free(void *p);
 /* Benchmark support: events[2i] and events[2i+1] (qg_event_create handles)
  * are recorded at the start and end of kernel i of this thread's
  * qg_moe_forward calls, timestamped by the dispatch itself
- * (hipExtLaunchKernelGGL).  Decode: 0 router, 1 routing, 2 gate/up, 3 down,
- * 4 combine.
- * Prefill: 0 router, 1 routing, 2 scan, 3 fill, 4 gate/up dense pass,
+ * (hipExtLaunchKernelGGL).  Decode kernels (up to 17 tokens, D of 2048 or 2560,
+ * F of 512 or 640, Q4_K gate/up, Q4_K or IQ4_NL down): 0 router, 1 routing, 2
+ * gate/up, 3 down, 4 combine.
+ * Prefill kernels (above 17 tokens; also up to 17 at D = 1024, F of 256, 512 or
+ * 640, in those formats with one down format): 0 router, 1 routing, 2 scan, 3 fill, 4 gate/up dense pass,
  * 5 gate/up other experts, 6 down dense pass, 7 down other experts,
  * 8 shared-expert down (when its format differs), 9 combine, 10 chunk
  * histogram (up to 256 tokens 2 covers 3 and 10 too).  n <= 32;
@@ -201,9 +208,10 @@ int qg_moe_kernel_events(void **events, int n);
 
 /* Benchmark support: record events[i] (qg_event_create handles) on the
  * launch stream at the phase boundaries of this thread's qg_moe_forward
- * calls: 0 start, 1 after the router, 2 after routing/dispatch, 3 after
- * gate/up, 4 after down, 5 after the combine (phases fused into one kernel
- * record adjacent events back to back).  n = 0 disables. */
+ * calls of up to 17 tokens that the decode kernels (see qg_moe_kernel_events)
+ * do not serve: 0 start, 1 after the router, 2 after routing/dispatch, 3 after
+ * gate/up, 4 after down, 5 after the combine.  The decode kernels and batches
+ * above 17 tokens record none.  n = 0 disables. */
 int qg_moe_phase_events(void **events, int n);
 
 /* Timing helpers for the benchmark (events on the calling thread's stream). */

@@ -32,6 +32,10 @@ extern "C" int qg_generic_forward(float *out, int *ids, float *weights, unsigned
 // `slot` of this thread's calls, if any.
 bool qg_kernel_event_pair(int slot, void **begin, void **end);
 
+// Records event i of qg_moe_phase_events on stream s, if the calling thread has
+// one registered.
+void qg_phase_mark(int i, hipStream_t s);
+
 // The prefill path of qg_moe_forward(_residual): 18..8192 tokens, and the decode
 // batches of qg_prefill_small_ok.
 bool qg_prefill_ok(const qg_moe_layer *L);

@@ -52,13 +52,9 @@ WsLayout ws_layout(int D, int F) {
     return L;
 }
 
-// Optional per-phase timing (benchmark support): events recorded on the
-// launch stream after each kernel of qg_moe_forward.
+// Optional per-phase timing (benchmark support, qg_phase_mark).
 thread_local void *tl_phase_ev[8] = {nullptr};
 thread_local int tl_phase_n = 0;
-void phase_mark(int i, hipStream_t s) {
-    if (i < tl_phase_n && tl_phase_ev[i]) (void)hipEventRecord((hipEvent_t)tl_phase_ev[i], s);
-}
 
 QG_DEV void route_token(int *s_ids, float *s_w, const float *s, int t, int lane, float *lds_v, int *lds_i) {
     qg_route_wave(s_ids + t * QG_TOP, s_w + t * QG_TOP, s, lane, lds_v, lds_i);
@@ -692,7 +688,7 @@ int launch_experts(const ExpertPhase &P, hipStream_t s) {
         gateup_mfma_kernel<3><<<dim3(gx, P.F / 64), 256, 0, s>>>(G);
         int rc = hipGetLastError();
         if (rc) return rc;
-        phase_mark(3, s);
+        qg_phase_mark(3, s);
         MfmaDown Dn{P.nt, P.D, P.F, maxa, P.down, P.sh_down, qg_row_bytes_host(P.dt, P.F),
                     P.sh_down ? qg_row_bytes_host(P.sdt, P.F) : 0, P.ds, P.midh, P.mids, P.route_w, P.slots, P.slots_out, MAXS};
         const int fs = P.sh_down ? P.sdt : P.dt;
@@ -702,13 +698,13 @@ int launch_experts(const ExpertPhase &P, hipStream_t s) {
         else if (fs == QT_IQ4_NL) down_mfma_kernel<QT_Q4_K, QT_IQ4_NL, 3><<<grid, 256, 0, s>>>(Dn);
         else down_mfma_kernel<QT_Q4_K, QT_Q4_K, 3><<<grid, 256, 0, s>>>(Dn);
         if ((rc = hipGetLastError())) return rc;
-        phase_mark(4, s);
+        qg_phase_mark(4, s);
         if (P.out) {
             const int quads = P.nt * P.D / 4;
             combine_kernel<<<(quads + 255) / 256, 256, 0, s>>>(P.out, P.slots, P.ds, P.sh_logit, P.ld, P.nt, P.D);
             rc = hipGetLastError();
         }
-        phase_mark(5, s);
+        qg_phase_mark(5, s);
         return rc;
     }
     const bool fast_gu = P.gt == QT_Q4_K && P.ut == QT_Q4_K && (!P.sh_gate || (P.sgt == QT_Q4_K && P.sut == QT_Q4_K)) &&
@@ -728,7 +724,7 @@ int launch_experts(const ExpertPhase &P, hipStream_t s) {
     }
     int rc = hipGetLastError();
     if (rc) return rc;
-    phase_mark(3, s);
+    qg_phase_mark(3, s);
     DownArgs D{P.nt, P.D, P.F, maxa, P.down, P.sh_down, qg_row_bytes_host(P.dt, P.F),
                P.sh_down ? qg_row_bytes_host(P.sdt, P.F) : 0, P.ds, P.mid, P.route_w, P.slots, P.slots_out};
     if (fast_dn) {
@@ -743,17 +739,21 @@ int launch_experts(const ExpertPhase &P, hipStream_t s) {
         down_generic_kernel<<<dim3(gx, (P.D + 1) / 2), 64, 0, s>>>(G);
     }
     if ((rc = hipGetLastError())) return rc;
-    phase_mark(4, s);
+    qg_phase_mark(4, s);
     if (P.out) {
         const int quads = P.nt * P.D / 4;
         combine_kernel<<<(quads + 255) / 256, 256, 0, s>>>(P.out, P.slots, P.ds, P.sh_logit, P.ld, P.nt, P.D);
         rc = hipGetLastError();
     }
-    phase_mark(5, s);
+    qg_phase_mark(5, s);
     return rc;
 }
 
 }  // namespace
+
+void qg_phase_mark(int i, hipStream_t s) {
+    if (i < tl_phase_n && tl_phase_ev[i]) (void)hipEventRecord((hipEvent_t)tl_phase_ev[i], s);
+}
 
 extern "C" {
 
@@ -790,7 +790,7 @@ int qg_generic_forward(float *out, int *ids, float *weights, unsigned char *flag
     float *logits = (float *)(ws + lay.logits);
     Disp *ds = (Disp *)(ws + lay.disp);
     const int rows = QG_EXPERTS + (sh ? 1 : 0);
-    phase_mark(0, s);
+    qg_phase_mark(0, s);
     int rc = qg_launch_matmul_exact(logits, (const uint8_t *)L->router, QT_F32, rows, D, x, nt,
                                     sh ? (const uint8_t *)L->sh_gate_inp : nullptr, s);
     if (rc) return rc;
@@ -798,13 +798,13 @@ int qg_generic_forward(float *out, int *ids, float *weights, unsigned char *flag
         logit_bias_kernel<<<nt, QG_EXPERTS, 0, s>>>(logits, rows, L->router_bias);
         if ((rc = hipGetLastError())) return rc;
     }
-    phase_mark(1, s);
+    qg_phase_mark(1, s);
     _Float16 *xh = (_Float16 *)(ws + lay.xh);
     float *xs = (float *)(ws + lay.xs);
     route_dispatch_kernel<<<1, RD_THREADS, 0, s>>>(ids, weights, flags, stats, logits, rows, nt, L->resident, L->threshold, ds,
                                                    sh ? 1 : 0, x, D, xh, xs);
     if ((rc = hipGetLastError())) return rc;
-    phase_mark(2, s);
+    qg_phase_mark(2, s);
     ExpertPhase P{x, nt, D, F, xh, xs, (_Float16 *)(ws + lay.midh), (float *)(ws + lay.mids),
                   (const uint8_t *)L->gate, (const uint8_t *)L->up, (const uint8_t *)L->down, L->gate_type, L->up_type, L->down_type,
                   sh ? (const uint8_t *)L->sh_gate : nullptr, sh ? (const uint8_t *)L->sh_up : nullptr,

@@ -1579,13 +1579,16 @@ int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsig
         if ((rc = hipGetLastError())) return rc;
         x = xn;
     }
+    const bool dec = nt <= QG_MAX_DECODE;   // a decode batch: group sums in fp32, phase events, no dense experts to split off
+    auto mark = [&](int phase) { if (dec) qg_phase_mark(phase, s); };
+    mark(0);
     // P1: router logits in the reference's order (+ bias)
     const XmArgs R{logits, rows, (const uint8_t *)L->router, (size_t)D * 4, QG_EXPERTS, D, x, nt, L->router_bias, 0, 0};
     if (nt >= 4096) pf_router<4, 2, 2, 2>(R, s);
     else if (xm_wide(QG_EXPERTS, nt)) pf_router<2, 2, 2, 4>(R, s);
     else pf_router<1, 1, 3, 4>(R, s);
     if ((rc = hipGetLastError())) return rc;
-    const bool dec = nt <= QG_MAX_DECODE;   // a decode batch: group sums in fp32, no dense experts to split off
+    mark(1);
     const int split = dec ? 0 : tl_pf_split;
     const bool i8 = split == 1;
     int8_t *xi8 = i8 ? (int8_t *)(ws + lay.xi8) : nullptr;
@@ -1609,6 +1612,7 @@ int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsig
                   (const int *)flag, nt, row_sx, (const float *)xsc);
         if ((rc = hipGetLastError())) return rc;
     }
+    mark(2);
     // grouped GEMMs: one launch over every group (dense experts, the shared
     // expert, the others); qg_prefill_int8_dense splits the dense experts off
     const int grid = qg_cu_count();
@@ -1631,6 +1635,7 @@ int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsig
     } else if ((rc = gate_up(0, 3, false, 5))) {
         return rc;
     }
+    mark(3);
     auto down = [&](int seg_lo, int seg_hi, int fmt, int slot) {
         DnArgs DA{nt, D, F, offsets, tt, seg_lo, seg_hi, row_slot, (const uint8_t *)L->down, sh ? (const uint8_t *)L->sh_down : nullptr,
                   qg_row_bytes_host(L->down_type, F), sh ? qg_row_bytes_host(L->sh_down_type, F) : 0, midp, msp, slots};
@@ -1649,6 +1654,7 @@ int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsig
         if ((rc = down(2, 3, L->down_type, 7))) return rc;
         if ((rc = down(1, 2, L->sh_down_type, 8))) return rc;
     }
+    mark(4);
     CombArgs CA{nt, D, ids, weights, flag, slots, sh ? logits + QG_EXPERTS : nullptr, rows, out, resid};
     pf_launch(9, pf_combine_kernel, dim3((D / 4 + 255) / 256, nt), dim3(256), 0, s, CA);
     if ((rc = hipGetLastError())) return rc;
@@ -1656,6 +1662,7 @@ int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsig
         pf_stats_kernel<<<1, 1024, 0, s>>>(stats, flag, (const int *)(ws + lay.missing), (const double *)(ws + lay.mass), nt);
         if ((rc = hipGetLastError())) return rc;
     }
+    mark(5);
     return hipSuccess;
 }
 

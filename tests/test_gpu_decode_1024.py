@@ -125,3 +125,22 @@ def test_decode_batch_independent(qgl, name):
     for nt in (1, 2, 3, 4, 9):
         got = P.forward(L, x[:nt]).out.get()[:nt]
         np.testing.assert_array_equal(got.view('u4'), whole[:nt].view('u4'), err_msg=f"{name} nt={nt}")
+
+
+@pytest.mark.parametrize("nt", [1, 2, 17])
+def test_decode_phase_events(qgl, nt):
+    """Every phase event is recorded, in order."""
+    L, _ = make("256-q4k")
+    events = [qgl.qg_event_create() for _ in range(6)]
+    try:
+        qg.call("moe_phase_events", (qg.C.c_void_p * 6)(*events), 6)
+        P.forward(L, synth.inputs(640, nt, 1024))
+        qg.call("moe_phase_events", None, 0)
+        for a, b in zip(events, events[1:]):
+            ms = qg.C.c_float(-1)
+            qg.call("event_elapsed", qg.C.byref(ms), a, b)
+            assert ms.value >= 0
+    finally:
+        qg.call("moe_phase_events", None, 0)
+        for e in events:
+            qgl.qg_event_destroy(e)
