@@ -202,7 +202,9 @@ void qg_host_free(void *p);
  * 640, in those formats with one down format): 0 router, 1 routing, 2 scan, 3 fill, 4 gate/up dense pass,
  * 5 gate/up other experts, 6 down dense pass, 7 down other experts,
  * 8 shared-expert down (when its format differs), 9 combine, 10 chunk
- * histogram (up to 256 tokens 2 covers 3 and 10 too).  n <= 32;
+ * histogram (up to 256 tokens 2 covers 3 and 10 too).  At D = 2560 (129..640
+ * tokens) and D = 1024 (385..896) gate/up is launched in two forms, 4 for long
+ * and 5 for short expert lists, of which one returns at once.  n <= 32;
  * n = 0 disables. */
 int qg_moe_kernel_events(void **events, int n);
 

@@ -65,8 +65,10 @@ constexpr int DENSE_MIN = 256;               // rows from which an expert is den
 // group gorder[p], whose tiles start at tbase[p]; tiles bounds[s] ..
 // bounds[s+1]-1 form segment s (0 dense, 1 shared, 2 the others).  mbase /
 // mbounds: the same prefixes of the row-tile counts M (a group of n rows has
-// ceil(n / 16) of them over its tiles).
-struct TileTable { int bounds[4]; int tbase[NG + 1]; int gorder[NG]; int mbase[NG + 1]; int mbounds[4]; };
+// ceil(n / 16) of them over its tiles).  tiles_gu, tiles_dn: whether the batch's
+// gate/up and down run on the 64-row tiles rather than the short-list kernels
+// (set where the launch leaves that to the device).
+struct TileTable { int bounds[4]; int tbase[NG + 1]; int gorder[NG]; int mbase[NG + 1]; int mbounds[4]; int tiles_gu, tiles_dn; };
 
 struct PfLayout {
     size_t logits, flag, missing, mass, xp, xsp, counts, offsets, tbase, row_token, row_slot, midp, msp, slots, xn, xi8, xsc,
@@ -237,9 +239,17 @@ QG_DEV int scan512(int v, int *s_tmp) {
     return v + base;
 }
 
+// Rows per tile unit (TM, in tiles of 8 rows) of the short-list kernels that a
+// batch's gate/up and down may take, 0 where nothing is left to decide.
+struct SpForms { int gu, dn; };
+
+// Price of a list of n rows on a short-list kernel with runs of 8 TM rows
+// (qg_sparse.h), in the same unit for any TM.
+QG_DEV int sp_price(int n, int tm) { return tm ? SP_C0 * ((n + 8 * tm - 1) / (8 * tm)) + (n + 7) / 8 : 0; }
+
 // The tile table of experts with n rows each (thread e: expert e; a 512-thread
 // block).
-QG_DEV void tile_table(TileTable *tt, int n, int shared_rows, int *s_tmp) {
+QG_DEV void tile_table(TileTable *tt, int n, int shared_rows, SpForms sp, int *s_tmp) {
     __shared__ int s_tiles[NG], s_m16[NG];
     __shared__ int s_wh[8][64], s_above[64];
     const int e = threadIdx.x;
@@ -285,8 +295,10 @@ QG_DEV void tile_table(TileTable *tt, int n, int shared_rows, int *s_tmp) {
     }
     __syncthreads();
     // prefixes over positions 0..511 (thread e: position e), then position 512
-    const int v = s_tiles[e], tincl = scan512(v, s_tmp);
-    const int m = s_m16[e], mincl = scan512(m, s_tmp);
+    // (tiles and row tiles share a scan: at most 1921 and 6145 at 8192 tokens)
+    const int v = s_tiles[e], m = s_m16[e], vm = scan512(m << 16 | v, s_tmp), tincl = vm & 0xffff, mincl = vm >> 16;
+    // both short-list prices in one scan (at most 1280 tokens: below 2^15 each)
+    const int price = sp.gu | sp.dn ? scan512(sp_price(n, sp.gu) << 16 | sp_price(n, sp.dn), s_tmp) : 0;  // block-uniform
     tt->tbase[e] = tincl - v;
     tt->mbase[e] = mincl - m;
     if (e == nd) {
@@ -318,12 +330,17 @@ QG_DEV void tile_table(TileTable *tt, int n, int shared_rows, int *s_tmp) {
         }
         tt->bounds[3] = all;
         tt->mbounds[3] = mall;
+        // 64-row tiles where their price (7 + 3 M per tile of M 16-row steps, as
+        // balanced_items) is below 5/3 of the short-list kernels'
+        const int tiles = 3 * (7 * all + 3 * mall);
+        tt->tiles_gu = sp.gu && tiles < 5 * ((price >> 16) + sp_price(shared_rows, sp.gu));
+        tt->tiles_dn = sp.dn && tiles < 5 * ((price & 0xffff) + sp_price(shared_rows, sp.dn));
     }
 }
 
 // tt may be null (dispatch only); with `status`, *status = OR of bad[0..nch).
 __global__ __launch_bounds__(512) void pf_scan_kernel(int *counts, int nch, int *offsets, TileTable *tt, int shared_rows,
-                                                      const int *bad, int *status) {
+                                                      SpForms sp, const int *bad, int *status) {
     __shared__ int s_tmp[8];
     const int e = threadIdx.x;
     if (status) {
@@ -357,7 +374,7 @@ __global__ __launch_bounds__(512) void pf_scan_kernel(int *counts, int nch, int 
         }
     }
     if (!tt) return;  // block-uniform
-    tile_table(tt, n, shared_rows, s_tmp);
+    tile_table(tt, n, shared_rows, sp, s_tmp);
 }
 
 // Histogram of an ids array alone (qg_moe_dispatch): chunk masks as in
@@ -423,7 +440,7 @@ __global__ __launch_bounds__(512) void pf_fill_kernel(int *row_token, int *row_s
 // workgroup looping over the selections was 0.7 longer.
 constexpr int PD_MAX = 256;
 constexpr int PD_SEL = PD_MAX * QG_TOP / 512;   // selections per thread
-__global__ __launch_bounds__(512) void pf_dispatch_kernel(int *offsets, TileTable *tt, int shared_rows, int *row_token, int *row_slot,
+__global__ __launch_bounds__(512) void pf_dispatch_kernel(int *offsets, TileTable *tt, int shared_rows, SpForms sp, int *row_token, int *row_slot,
                                                           const int *ids, const int *flag, int nt, float *row_sx, const float *xsc) {
     constexpr int NCH = PD_MAX / PF_CHUNK;
     __shared__ uint32_t s_mask[NCH][QG_EXPERTS];
@@ -466,7 +483,7 @@ __global__ __launch_bounds__(512) void pf_dispatch_kernel(int *offsets, TileTabl
         row_slot[pos] = i;
         if (row_sx) row_sx[pos] = xsc[t];
     }
-    if (tt) tile_table(tt, n, shared_rows, s_tmp);  // block-uniform
+    if (tt) tile_table(tt, n, shared_rows, sp, s_tmp);  // block-uniform
 }
 
 // ---------------- GEMM building blocks ----------------
@@ -607,6 +624,7 @@ struct GuArgs {
     _Float16 *midp, *msp;            // [rows][2][F] (down format order), [rows][2][F/32]
     int down_fmt, sh_down_fmt;
     const int8_t *xi8; const float *xsc, *row_sx;   // the int8 variant: planes [nt][2][D], scale per token and per CSR row
+    const int *only;                 // if not null, run only where *only is set (TileTable::tiles_gu)
 };
 
 // (the kernel follows the down kernels: it shares their 128-element stage)
@@ -689,7 +707,7 @@ QG_DEV void iq_chunk_lds(qg_f4 (&y)[MY][NCT], const uint8_t *slot, const int (&d
 // block as two column tiles.  Steps are the item's K chunks of 128.  As in
 // the gate/up kernel, the step loop runs inside one instantiation per row-tile
 // count, and the per-lane copy addresses are formed once per item.
-__global__ __launch_bounds__(512, 1) void pf_down_iq_kernel(DnArgs A) {
+QG_DEV void down_tiles_iq(const DnArgs &A) {
     extern __shared__ uint4 s_dyn[];
     uint8_t *lds = (uint8_t *)s_dyn;
     __shared__ int s_tb[NG + 1], s_go[NG], s_off[QG_EXPERTS + 1];
@@ -1037,15 +1055,24 @@ QG_DEV void gq_chunk(qg_f4 (&y)[MY][NC], const uint8_t *slot, const uint8_t *st,
 // instantiation per row-tile count M, entered once per item, so the
 // accumulators stay in place for the item's steps; the per-lane addresses of
 // the copies are formed once per item and advanced per step.
+struct GuShared {
+    int2 it[IT_RING];
+    int tb[NG + 1], go[NG], off[QG_EXPERTS + 1];
+    int src[2][PT];
+    float sx[2][PT];          // the int8 variant: row scales of the item's rows
+    float gs[PF_WAVES][PT];   // 16-row partial sums of the 32-row groups (Q4_K down format)
+};
 template <bool I8>
-__global__ __launch_bounds__(512, 1) void pf_gateup_kernel(GuArgs A) {
+QG_DEV void gateup_tiles(const GuArgs &A, GuShared &S) {
     extern __shared__ uint4 s_dyn[];
     uint8_t *lds = (uint8_t *)s_dyn;
-    __shared__ int s_tb[NG + 1], s_go[NG], s_off[QG_EXPERTS + 1];
-    __shared__ int2 s_it[IT_RING];
-    __shared__ int s_src[2][PT];
-    __shared__ float s_sx[2][PT];            // the int8 variant: row scales of the item's rows
-    __shared__ float s_gs[PF_WAVES][PT];     // 16-row partial sums of the 32-row groups (Q4_K down format)
+    auto &s_tb = S.tb;
+    auto &s_off = S.off;
+    auto &s_go = S.go;
+    auto &s_it = S.it;
+    auto &s_src = S.src;
+    auto &s_sx = S.sx;
+    auto &s_gs = S.gs;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, j = lane & 15, kq = lane >> 4;
     for (int i = tid; i <= NG; i += 512) {
         s_tb[i] = A.tt->tbase[i];
@@ -1239,6 +1266,12 @@ __global__ __launch_bounds__(512, 1) void pf_gateup_kernel(GuArgs A) {
     }
 }
 
+template <bool I8>
+__global__ __launch_bounds__(512, 1) void pf_gateup_kernel(GuArgs A) {
+    __shared__ GuShared S;
+    if (!A.only || *A.only) gateup_tiles<I8>(A, S);  // block-uniform
+}
+
 // Q4_K down over half-superblock steps, as the gate/up kernel: item = (group,
 // 64-row tile, 256 D rows); wave w: D rows 32 w .. +31 of the block as two column
 // tiles, their bytes through the wave's own ring; the mid rows (CSR order) staged
@@ -1246,7 +1279,7 @@ __global__ __launch_bounds__(512, 1) void pf_gateup_kernel(GuArgs A) {
 // row-tile count.  Against the kernel this replaces (weights in registers, a
 // test per row tile, 256-column steps): 698 -> 540 us at 8192
 // tokens (F 512), 59 -> 49 at 1500 (F 256).
-__global__ __launch_bounds__(512, 1) void pf_down_kernel(DnArgs A) {
+QG_DEV void down_tiles_q4k(const DnArgs &A) {
     extern __shared__ uint4 s_dyn[];
     uint8_t *lds = (uint8_t *)s_dyn;
     __shared__ int s_tb[NG + 1], s_go[NG], s_off[QG_EXPERTS + 1];
@@ -1386,10 +1419,35 @@ __global__ __launch_bounds__(512, 1) void pf_down_kernel(DnArgs A) {
     }
 }
 
+__global__ __launch_bounds__(512, 1) void pf_down_iq_kernel(DnArgs A) { down_tiles_iq(A); }
+__global__ __launch_bounds__(512, 1) void pf_down_kernel(DnArgs A) { down_tiles_q4k(A); }
+
+// Both forms in one launch: the short-list kernel or, where the lists are long
+// (*S.tiles), the 64-row tiles, whose small arrays lie after their stages.
+constexpr int GU_PICK_LDS = SpGu<8, 3>::LDS;
+static_assert(PF_GQ_LDS + sizeof(GuShared) <= GU_PICK_LDS, "both forms fit");
+__global__ __launch_bounds__(512, 1) void pf_gateup_pick_kernel(SpGuArgs S, GuArgs T) {
+    extern __shared__ uint4 s_dyn[];
+    if (!gateup_sp<8, 3, false>(S)) gateup_tiles<false>(T, *(GuShared *)((uint8_t *)s_dyn + PF_GQ_LDS));  // block-uniform
+}
+template <int FMT, int NB>
+constexpr int dn_pick_lds() {
+    constexpr int t = FMT == QT_Q4_K ? PF_GQ_LDS : PF_IQ_LDS, s = SpDn<FMT, NB>::LDS;
+    return t > s ? t : s;
+}
+template <int FMT, int NB, int TM>
+__global__ __launch_bounds__(512, 1) void pf_down_pick_kernel(SpDnArgs S, DnArgs T) {
+    if (down_sp<FMT, NB, TM, false>(S)) return;  // block-uniform
+    if constexpr (FMT == QT_Q4_K) down_tiles_q4k(T);
+    else down_tiles_iq(T);
+}
+
 // The kernels of qg_sparse.h for batches whose experts have few rows, where
 // they stream and convert the weights in fewer instructions; above, the 64-row
-// tiles of pf_gateup_kernel and the down kernels re-read no weights.  The batch
-// limits lie where the two cross (uniform routing, us, 64-row tiles / these):
+// tiles of pf_gateup_kernel and the down kernels re-read no weights.
+//
+// Two rules choose.  First, by batch size: the short-list kernels run up to the
+// sizes where the two cross under uniform routing (us, 64-row tiles / these):
 //   gate/up D 2048: 40 tokens 111 / 67, 400 194 / 144, 1000 245 / 204, 1500 284 / 300
 //           D 2560: 60 tokens 200 / 147, 301 283 / 221, 600 297 / 271, 1200 366 / 471
 //           D 1024: 100 tokens 54 / 37, 600 66 / 53, 1500 80 / 97
@@ -1398,34 +1456,74 @@ __global__ __launch_bounds__(512, 1) void pf_down_kernel(DnArgs A) {
 //        IQ4_NL F 512: 40 tokens 71 / 48, 400 127 / 117, 500 127 / 129
 //               F 640: 60 tokens 131 / 89, 301 185 / 139, 400 184 / 170, 600 197 / 233
 //               F 256: 100 tokens 35 / 28, 600 45 / 41, 1500 59 / 76
+// Second, below those sizes, by the rows of the lists, which only the device
+// knows: tokens of one context share their experts, and a list of n rows is
+// converted n / 24 or n / 16 times (IQ4_NL down: n / 8) against n / 64.
+// tile_table compares the two forms' prices over the batch's lists.  The factor
+// 5/3 comes from times of both over 18..1280 tokens of uniform, Zipf, loosely
+// and closely related tokens, every shape above (336 points): the rule's choice is
+// on average 0.4 % and at most 12 % behind the better one, always the short-list
+// kernel 14 % (2048/512 IQ4_NL, 448 closely related tokens: gate/up 82 / 73 us, down
+// 91 / 40; 2560/640: 146 / 90, 133 / 62).  Where both forms have the same
+// workgroups they are one kernel; gate/up at D = 2560 and 1024, whose short-list
+// kernels have 640 and 256 threads, takes two launches of which one is idle (2.5
+// us), from the batch on at which the tiles can be ahead by more than that.
+//
 // Runs of two tiles hold the mid fragments of K = 512 in registers for Q4_K; the
 // IQ4_NL conversion needs the registers, so it takes one tile there (with two,
 // spills in the loop made 400 tokens 262 us).  Decode batches (qg_prefill_small_ok)
 // take the FULL forms.
-bool pf_gateup_sp(const SpGuArgs &A, int cus, hipStream_t s) {
-    if (A.D == 1024 && A.nt <= QG_MAX_DECODE) pf_launch(5, pf_gateup_sp_kernel<4, 2, true>, dim3(2 * cus), dim3(256), SpGu<4, 2>::LDS, s, A);
-    else if (A.D == 2048 && A.nt <= 1280) pf_launch(5, pf_gateup_sp_kernel<8, 3, false>, dim3(cus), dim3(512), SpGu<8, 3>::LDS, s, A);
-    else if (A.D == 2560 && A.nt <= 640) pf_launch(5, pf_gateup_sp_kernel<10, 2, false>, dim3(cus), dim3(640), SpGu<10, 2>::LDS, s, A);
-    else if (A.D == 1024 && A.nt <= 896) pf_launch(5, pf_gateup_sp_kernel<4, 2, false>, dim3(2 * cus), dim3(256), SpGu<4, 2>::LDS, s, A);
-    else return false;
-    return true;
+constexpr int sp_down_tm(int fmt, int nb) { return fmt == QT_IQ4_NL && nb >= 16 ? 1 : 2; }
+SpForms sp_forms(int D, int F, int down_fmt, int nt) {
+    SpForms f{0, 0};
+    if (D == 2048 && nt <= 1280) f.gu = 3;
+    if ((D == 2560 && nt <= 640) || (D == 1024 && nt <= 896)) f.gu = 2;
+    const int most = down_fmt == QT_Q4_K ? (F == 256 ? 768 : F == 512 ? 1280 : 0) : (F == 256 ? 640 : F == 512 || F == 640 ? 448 : 0);
+    if (nt <= most) f.dn = sp_down_tm(down_fmt, F / 32);
+    return f;
 }
-bool pf_down_sp(const SpDnArgs &A, int fmt, int F, int cus, hipStream_t s) {
-    auto go = [&](auto FC, auto NC, int most) {
-        constexpr int FMT = decltype(FC)::value, NB = decltype(NC)::value, TM = FMT == QT_IQ4_NL && NB >= 16 ? 1 : 2;
-        if (A.nt > most) return false;
-        constexpr bool SUMS = FMT == QT_Q4_K;   // IQ4_NL has no min term
-        if (A.nt <= QG_MAX_DECODE) pf_launch(7, pf_down_sp_kernel<FMT, NB, TM, SUMS>, dim3(cus), dim3(512), SpDn<FMT, NB>::LDS, s, A);
-        else pf_launch(7, pf_down_sp_kernel<FMT, NB, TM, false>, dim3(cus), dim3(512), SpDn<FMT, NB>::LDS, s, A);
-        return true;
+// The forms of which the device chooses by the lists.
+SpForms sp_ask(const SpForms &f, int D, int nt) {
+    return SpForms{nt > (D >= 2048 ? 128 : 384) ? f.gu : 0, nt > 64 ? f.dn : 0};
+}
+// gate/up where sp_forms(...).gu is not 0
+int pf_gateup_sp(const SpGuArgs &A, const GuArgs &T, int cus, hipStream_t s) {
+    const bool dec = A.nt <= QG_MAX_DECODE;
+    if (A.D == 2048) {
+        pf_launch(5, pf_gateup_pick_kernel, dim3(cus), dim3(512), GU_PICK_LDS, s, A, T);
+        return hipGetLastError();
+    }
+    if (A.D == 2560) pf_launch(5, pf_gateup_sp_kernel<10, 2, false>, dim3(cus), dim3(640), SpGu<10, 2>::LDS, s, A);
+    else if (dec) pf_launch(5, pf_gateup_sp_kernel<4, 2, true>, dim3(2 * cus), dim3(256), SpGu<4, 2>::LDS, s, A);
+    else pf_launch(5, pf_gateup_sp_kernel<4, 2, false>, dim3(2 * cus), dim3(256), SpGu<4, 2>::LDS, s, A);
+    const int rc = hipGetLastError();
+    if (rc || !A.tiles) return rc;
+    pf_launch(4, pf_gateup_kernel<false>, dim3(cus), dim3(512), PF_GQ_LDS, s, T);
+    return hipGetLastError();
+}
+// down where sp_forms(...).dn is not 0
+int pf_down_sp(const SpDnArgs &A, const DnArgs &T, int fmt, int cus, hipStream_t s) {
+    auto go = [&](auto FC, auto NC) {
+        constexpr int FMT = decltype(FC)::value, NB = decltype(NC)::value, TM = sp_down_tm(FMT, NB);
+        if constexpr (FMT == QT_Q4_K) {   // (IQ4_NL has no min term)
+            if (A.nt <= QG_MAX_DECODE) {
+                pf_launch(7, pf_down_sp_kernel<FMT, NB, TM, true>, dim3(cus), dim3(512), SpDn<FMT, NB>::LDS, s, A);
+                return;
+            }
+        }
+        pf_launch(7, pf_down_pick_kernel<FMT, NB, TM>, dim3(cus), dim3(512), dn_pick_lds<FMT, NB>(), s, A, T);
     };
     using Q4 = std::integral_constant<int, QT_Q4_K>;
     using IQ = std::integral_constant<int, QT_IQ4_NL>;
     using N8 = std::integral_constant<int, 8>;
     using N16 = std::integral_constant<int, 16>;
     using N20 = std::integral_constant<int, 20>;
-    if (fmt == QT_Q4_K) return F == 256 ? go(Q4{}, N8{}, 768) : F == 512 ? go(Q4{}, N16{}, 1280) : false;
-    return F == 256 ? go(IQ{}, N8{}, 640) : F == 512 ? go(IQ{}, N16{}, 448) : F == 640 ? go(IQ{}, N20{}, 448) : false;
+    if (fmt == QT_Q4_K && T.F == 256) go(Q4{}, N8{});
+    else if (fmt == QT_Q4_K) go(Q4{}, N16{});
+    else if (T.F == 256) go(IQ{}, N8{});
+    else if (T.F == 512) go(IQ{}, N16{});
+    else go(IQ{}, N20{});
+    return hipGetLastError();
 }
 
 // ---------------- P7: combine ----------------
@@ -1598,14 +1696,20 @@ int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsig
                  sh ? L->sh_gate_inp : nullptr, logits + QG_EXPERTS, xi8, xsc};
     pf_launch(1, pf_route_kernel, dim3((nt + 3) / 4), dim3(512), 0, s, RA);
     if ((rc = hipGetLastError())) return rc;
+    // gate/up and down on the short-list kernels, on the 64-row tiles, or as the lists turn out
+    const bool one_fmt = !sh || L->sh_down_type == L->down_type;
+    SpForms form = sp_forms(D, F, L->down_type, nt);
+    if (split) form.gu = 0;
+    if (!one_fmt) form.dn = 0;
+    const SpForms ask = sp_ask(form, D, nt);
     if (nt <= PD_MAX) {
-        pf_launch(2, pf_dispatch_kernel, dim3(1), dim3(512), 0, s, offsets, tt, sh ? nt : 0, row_token, row_slot,
+        pf_launch(2, pf_dispatch_kernel, dim3(1), dim3(512), 0, s, offsets, tt, sh ? nt : 0, ask, row_token, row_slot,
                   (const int *)ids, (const int *)flag, nt, row_sx, (const float *)xsc);
         if ((rc = hipGetLastError())) return rc;
     } else {
         pf_launch(10, pf_count_kernel, dim3(nch), dim3(512), 0, s, counts, (int *)nullptr, (const int *)ids, (const int *)flag, nt);
         if ((rc = hipGetLastError())) return rc;
-        pf_launch(2, pf_scan_kernel, dim3(1), dim3(512), 0, s, counts, nch, offsets, tt, sh ? nt : 0, (const int *)nullptr,
+        pf_launch(2, pf_scan_kernel, dim3(1), dim3(512), 0, s, counts, nch, offsets, tt, sh ? nt : 0, ask, (const int *)nullptr,
                   (int *)nullptr);
         if ((rc = hipGetLastError())) return rc;
         pf_launch(3, pf_fill_kernel, dim3(nch), dim3(512), 0, s, row_token, row_slot, (const int *)counts, (const int *)ids,
@@ -1616,19 +1720,23 @@ int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsig
     // grouped GEMMs: one launch over every group (dense experts, the shared
     // expert, the others); qg_prefill_int8_dense splits the dense experts off
     const int grid = qg_cu_count();
+    const int *tiles_gu = ask.gu ? &tt->tiles_gu : nullptr, *tiles_dn = ask.dn ? &tt->tiles_dn : nullptr;
+    auto gu_args = [&](int seg_lo, int seg_hi) {
+        return GuArgs{nt, D, F, offsets, tt, seg_lo, seg_hi, row_token, (const uint8_t *)L->gate, (const uint8_t *)L->up,
+                      sh ? (const uint8_t *)L->sh_gate : nullptr, sh ? (const uint8_t *)L->sh_up : nullptr, qg_row_bytes_host(QT_Q4_K, D),
+                      xp, xsp, midp, msp, L->down_type, sh ? L->sh_down_type : L->down_type, xi8, xsc, row_sx, tiles_gu};
+    };
     auto gate_up = [&](int seg_lo, int seg_hi, bool int8, int slot) {
-        GuArgs G{nt, D, F, offsets, tt, seg_lo, seg_hi, row_token, (const uint8_t *)L->gate, (const uint8_t *)L->up,
-                 sh ? (const uint8_t *)L->sh_gate : nullptr, sh ? (const uint8_t *)L->sh_up : nullptr, qg_row_bytes_host(QT_Q4_K, D),
-                 xp, xsp, midp, msp, L->down_type, sh ? L->sh_down_type : L->down_type, xi8, xsc, row_sx};
+        const GuArgs G = gu_args(seg_lo, seg_hi);
         if (int8) pf_launch(slot, pf_gateup_kernel<true>, dim3(grid), dim3(512), PF_GQ_LDS, s, G);
         else pf_launch(slot, pf_gateup_kernel<false>, dim3(grid), dim3(512), PF_GQ_LDS, s, G);
         return hipGetLastError();
     };
-    const SpGuArgs GS{nt, D, F, offsets, row_token, (const uint8_t *)L->gate, (const uint8_t *)L->up,
-                      sh ? (const uint8_t *)L->sh_gate : nullptr, sh ? (const uint8_t *)L->sh_up : nullptr, qg_row_bytes_host(QT_Q4_K, D),
-                      xp, xsp, midp, msp, L->down_type, sh ? L->sh_down_type : L->down_type};
-    if (!split && pf_gateup_sp(GS, grid, s)) {
-        if ((rc = hipGetLastError())) return rc;
+    if (form.gu) {
+        const SpGuArgs GS{nt, D, F, offsets, row_token, (const uint8_t *)L->gate, (const uint8_t *)L->up,
+                          sh ? (const uint8_t *)L->sh_gate : nullptr, sh ? (const uint8_t *)L->sh_up : nullptr,
+                          qg_row_bytes_host(QT_Q4_K, D), xp, xsp, midp, msp, L->down_type, sh ? L->sh_down_type : L->down_type, tiles_gu};
+        if ((rc = pf_gateup_sp(GS, gu_args(0, 3), grid, s))) return rc;
     } else if (split) {
         if ((rc = gate_up(0, 1, i8, 4))) return rc;
         if ((rc = gate_up(1, 3, false, 5))) return rc;
@@ -1636,17 +1744,19 @@ int qg_prefill_forward(float *out, float *resid, int *ids, float *weights, unsig
         return rc;
     }
     mark(3);
+    auto dn_args = [&](int seg_lo, int seg_hi) {
+        return DnArgs{nt, D, F, offsets, tt, seg_lo, seg_hi, row_slot, (const uint8_t *)L->down, sh ? (const uint8_t *)L->sh_down : nullptr,
+                      qg_row_bytes_host(L->down_type, F), sh ? qg_row_bytes_host(L->sh_down_type, F) : 0, midp, msp, slots};
+    };
     auto down = [&](int seg_lo, int seg_hi, int fmt, int slot) {
-        DnArgs DA{nt, D, F, offsets, tt, seg_lo, seg_hi, row_slot, (const uint8_t *)L->down, sh ? (const uint8_t *)L->sh_down : nullptr,
-                  qg_row_bytes_host(L->down_type, F), sh ? qg_row_bytes_host(L->sh_down_type, F) : 0, midp, msp, slots};
+        const DnArgs DA = dn_args(seg_lo, seg_hi);
         if (fmt == QT_Q4_K) pf_launch(slot, pf_down_kernel, dim3(grid), dim3(512), PF_GQ_LDS, s, DA);
         else pf_launch(slot, pf_down_iq_kernel, dim3(grid), dim3(512), PF_IQ_LDS, s, DA);
         return hipGetLastError();
     };
-    const bool one_fmt = !sh || L->sh_down_type == L->down_type;
-    const SpDnArgs DS{nt, D, offsets, row_slot, (const uint8_t *)L->down, sh ? (const uint8_t *)L->sh_down : nullptr, midp, msp, slots};
-    if (one_fmt && pf_down_sp(DS, L->down_type, F, grid, s)) {
-        if ((rc = hipGetLastError())) return rc;
+    if (form.dn) {
+        const SpDnArgs DS{nt, D, offsets, row_slot, (const uint8_t *)L->down, sh ? (const uint8_t *)L->sh_down : nullptr, midp, msp, slots, tiles_dn};
+        if ((rc = pf_down_sp(DS, dn_args(0, 3), L->down_type, grid, s))) return rc;
     } else if (one_fmt) {
         if ((rc = down(0, 3, L->down_type, 7))) return rc;
     } else {  // the shared expert's down in its own format
@@ -1680,7 +1790,7 @@ int qg_prefill_dispatch(int *offsets, int *row_token, int *row_slot, int *status
     pf_count_kernel<<<nch, 512, 0, s>>>(counts, bad, ids, nullptr, nt);
     int rc = hipGetLastError();
     if (rc) return rc;
-    pf_scan_kernel<<<1, 512, 0, s>>>(counts, nch, offsets, nullptr, 0, bad, status);
+    pf_scan_kernel<<<1, 512, 0, s>>>(counts, nch, offsets, nullptr, 0, SpForms{0, 0}, bad, status);
     if ((rc = hipGetLastError())) return rc;
     pf_fill_kernel<<<nch, 512, 0, s>>>(row_token, row_slot, counts, ids, nullptr, nt, nullptr, nullptr);
     return hipGetLastError();

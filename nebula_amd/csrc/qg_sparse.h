@@ -205,22 +205,27 @@ struct SpGuArgs {
     const _Float16 *xp, *xsp;
     _Float16 *midp, *msp;            // [rows][2][F] (down format order), [rows][2][F/32] (FULL: fp32 [rows][F/32], as xsp)
     int down_fmt, sh_down_fmt;
+    const int *tiles;                // if not null, *tiles: the 64-row tiles have the batch
 };
 
+// Returns false, with nothing done, where the 64-row tiles have the batch.
 template <int W, int TM, bool FULL>
-__global__ __launch_bounds__(64 * W, 1) void pf_gateup_sp_kernel(SpGuArgs A) {
+QG_DEV bool gateup_sp(const SpGuArgs &A) {
     extern __shared__ uint4 s_dyn[];
     __shared__ SpList S;
     __shared__ int s_off[QG_EXPERTS + 1];
     __shared__ float s_gs[W][4];   // 16-row sums of the jobs' tile rows (Q4_K down format)
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, j = lane & 15, kq = lane >> 4;
+    const int tiles = A.tiles ? *A.tiles : 0;   // arrives with the offsets
     for (int i = tid; i <= QG_EXPERTS; i += 64 * W) s_off[i] = A.offsets[i];
     __syncthreads();
+    if (tiles) return false;
     using MIN = SpMin<FULL>;
     const int D = A.D, F = A.F, nsr = F / 16;   // sub-units per run
+    const int fmts = A.down_fmt | A.sh_down_fmt << 8;   // (chosen between by address, they keep A in scratch)
     sp_build<64 * W, TM>(S, s_dyn, s_off, A.nt, A.sh_gate != nullptr, F / 32, sp_part(), gridDim.x);
     const int nsub = 2 * __builtin_amdgcn_readfirstlane(S.pos[1][3] - S.pos[0][3]);
-    if (nsub <= 0) return;  // block-uniform
+    if (nsub <= 0) return true;  // block-uniform
     uint4 *ring = s_dyn + (size_t)wave * 3 * SP_SLOT;
     float2 *red = (float2 *)(s_dyn + SpGu<W, TM>::RING / 16);
 
@@ -289,7 +294,7 @@ __global__ __launch_bounds__(64 * W, 1) void pf_gateup_sp_kernel(SpGuArgs A) {
             for (int f = 0; f < 8; f++) sp_pin(af[m][f]);
             sp_pin(sf[m]);
         }
-        const int fmt = sh ? A.sh_down_fmt : A.down_fmt;
+        const int fmt = (fmts >> (sh ? 8 : 0)) & 0xff;
         constexpr int NB = SpGu<W, TM>::batch(M);
         constexpr bool TWO = NB == 1 && SpGu<W, TM>::TS >= 2 * M;   // sub-units alternate between two sum buffers
         float half = 0.0f;   // NB == 1: the first 16 rows' sum of the unit's 32-row group
@@ -369,6 +374,12 @@ __global__ __launch_bounds__(64 * W, 1) void pf_gateup_sp_kernel(SpGuArgs A) {
         sub = 0;
         if (++tau == R.runs) { tau = 0; x++; }
     }
+    return true;
+}
+
+template <int W, int TM, bool FULL>
+__global__ __launch_bounds__(64 * W, 1) void pf_gateup_sp_kernel(SpGuArgs A) {
+    gateup_sp<W, TM, FULL>(A);
 }
 
 // ---- down: a wave per 16 output rows ----
@@ -393,23 +404,27 @@ struct SpDnArgs {
     const uint8_t *down, *sh_down;   // rows of FMT, the shared expert's too
     const _Float16 *midp, *msp;
     float *slots;                    // [rows][D]: slot t*10+k, shared rows at nt*10+t
+    const int *tiles;                // as SpGuArgs
 };
 
+// Returns false, with nothing done, where the 64-row tiles have the batch.
 template <int FMT, int NB, int TM, bool FULL>
-__global__ __launch_bounds__(512, 1) void pf_down_sp_kernel(SpDnArgs A) {
+QG_DEV bool down_sp(const SpDnArgs &A) {
     using C = SpDn<FMT, NB>;
     constexpr int F = 32 * NB, RB = C::RB, CP = C::CP;
     extern __shared__ uint4 s_dyn[];
     __shared__ SpList S;
     __shared__ int s_off[QG_EXPERTS + 1];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, j = lane & 15, kq = lane >> 4;
+    const int tiles = A.tiles ? *A.tiles : 0;   // arrives with the offsets
     for (int i = tid; i <= QG_EXPERTS; i += 512) s_off[i] = A.offsets[i];
     __syncthreads();
+    if (tiles) return false;
     const int D = A.D, units = D / 16;
     static_assert(C::LDS >= SP_SCRATCH, "the build's scratch fits the rings");
     sp_build<512, TM>(S, s_dyn, s_off, A.nt, A.sh_down != nullptr, units, sp_part(), gridDim.x);
     const int mine = __builtin_amdgcn_readfirstlane(S.pos[1][3] - S.pos[0][3]) - wave;   // this wave: units wave, wave + 8, ...
-    if (mine <= 0) return;  // no block barrier from here on
+    if (mine <= 0) return true;  // no block barrier from here on
     const int nu = (mine + 7) / 8;
     uint8_t *ring = (uint8_t *)s_dyn + (size_t)wave * 3 * C::SLOT;
     uint32_t c_off[CP];
@@ -558,4 +573,8 @@ __global__ __launch_bounds__(512, 1) void pf_down_sp_kernel(SpDnArgs A) {
         settle(x, tau, u, R);
     }
     wait_vmem();  // no copy may land in shared memory after the workgroup ends
+    return true;
 }
+
+template <int FMT, int NB, int TM, bool FULL>
+__global__ __launch_bounds__(512, 1) void pf_down_sp_kernel(SpDnArgs A) { down_sp<FMT, NB, TM, FULL>(A); }
