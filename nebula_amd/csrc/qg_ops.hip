@@ -251,9 +251,13 @@ void launch_xm(float *out, const uint8_t *w, int rows, int cols, const float *x,
             return;
         }
     }
-    constexpr int CH = TYPE == QT_F32 ? 1 : 2, XR = TYPE == QT_F32 ? 3 : 2;  // F32 rows may be an odd number of chunks
-    if (nt > 16 && nt <= 20) xm_run<TYPE, 1, 1, 1, CH, XR, 4, 4>(A, s);
-    else xm_run<TYPE, 1, 0, 1, CH, XR, 4, 4>(A, s);
+    if constexpr (TYPE == QT_F32) {  // rows may be an odd number of chunks; 20-token tiles lose (512 x 2048: 10.0 against 7.6 us)
+        xm_run<TYPE, 1, 0, 1, 1, 3, 4, 4>(A, s);
+        return;
+    } else {
+        if (nt > 16 && nt <= 20) xm_run<TYPE, 1, 1, 1, 2, 2, 4, 4>(A, s);
+        else xm_run<TYPE, 1, 0, 1, 2, 2, 4, 4>(A, s);
+    }
 }
 
 template <int TYPE>
@@ -278,9 +282,15 @@ void launch_mm_exact(float *out, const uint8_t *w, int type, int rows, int cols,
         if (aligned && cols % 256 == 0) { launch_xm<TYPE>(out, w, rows, cols, x, nt, stride, s); return; }
     }
     if constexpr (TYPE == QT_F32) {
-        // 32 tokens and fewer: too few tiles of the router's 512 rows (512 x
-        // 2048: 17 tokens 5.3 against 9.3 us, 40 tokens 8.3 against 6.8)
-        if (aligned && cols % 128 == 0 && nt > 32) { launch_xm<TYPE>(out, w, rows, cols, x, nt, stride, s); return; }
+        // A tile's time does not fall with its outputs, the vector chains' does:
+        // with few outputs they are the faster (2048 columns, us, chains / tiles:
+        // 16 x 64 tokens 4.8 / 7.4, 256 x 40 6.5 / 7.5, 256 x 64 7.9 / 7.6, 512 x 24
+        // 6.9 / 7.6, 512 x 32 7.9 / 7.6, 1024 x 12 6.8 / 7.6, 2560 x 8 9.3 / 7.7), up to
+        // 64 tokens; above, they hold 16 tokens per wave and take 69 us.
+        if (aligned && cols % 128 == 0 && nt > 1 && (nt > 64 || (long)rows * nt > 12288)) {
+            launch_xm<TYPE>(out, w, rows, cols, x, nt, stride, s);
+            return;
+        }
     }
     dim3 grid((rows + 1) / 2, 1);
     if (nt == 1) { mm_exact_kernel<TYPE, 1><<<grid, 64, 0, s>>>(out, w, type, rows, cols, x, nt, stride, extra); return; }

@@ -1,0 +1,64 @@
+"""qg_matmul's choice of kernels by size.  Each form gives the reference's bits,
+so the batches on both sides of every limit are compared with the oracle bit
+for bit; and where a size had been sent to the slower form, its time is held
+against that of a size that has always been on the faster one."""
+import sys
+
+import numpy as np
+import pytest
+
+import oracle as O
+from nebula_amd import qg
+from nebula_amd.qg import Device, call
+from test_gpu_exact_tiles import run
+from test_oracle_cpu import legal_blocks
+
+pytestmark = pytest.mark.gpu
+
+
+def check(typ, rows, cols, tokens):
+    rng = np.random.default_rng(100 * typ + rows + cols)
+    w = np.ascontiguousarray(legal_blocks(rng, typ, rows, cols))
+    for nt in tokens:
+        print(f"matmul route type={typ} {rows}x{cols} nt={nt}", flush=True, file=sys.stderr)
+        x = rng.normal(0, .5, (nt, cols)).astype(np.float32)
+        np.testing.assert_array_equal(run(typ, w, rows, cols, x).view('u4'), O.matmul(w, typ, rows, cols, x).view('u4'),
+                                      err_msg=f"type {typ} {rows}x{cols} nt {nt}")
+
+
+def graph_us(typ, rows, cols, nt):
+    """Time of one call in a graph of 20, the least of 15 replays."""
+    lib = qg.lib()
+    w, x, out = Device(nbytes=rows * qg.row_bytes(typ, cols)), Device(nbytes=nt * cols * 4), Device(nbytes=nt * rows * 4)
+    begin, end, graph = lib.qg_event_create(), lib.qg_event_create(), qg.C.c_void_p()
+    best = float("inf")
+    call("matmul", out.p, w.p, typ, rows, cols, x.p, nt)
+    call("graph_begin", qg.C.byref(graph))
+    for _ in range(20):
+        call("matmul", out.p, w.p, typ, rows, cols, x.p, nt)
+    call("graph_end", graph)
+    try:
+        for _ in range(15):
+            call("event_record", begin)
+            call("graph_launch", graph)
+            call("event_record", end)
+            call("sync")
+            ms = qg.C.c_float()
+            call("event_elapsed", qg.C.byref(ms), begin, end)
+            best = min(best, ms.value * 1e3 / 20)
+    finally:
+        lib.qg_graph_destroy(graph)
+        lib.qg_event_destroy(begin)
+        lib.qg_event_destroy(end)
+    print(f"matmul type={typ} {rows}x{cols} nt={nt}: {best:.2f} us", flush=True, file=sys.stderr)
+    return best
+
+
+@pytest.mark.parametrize("rows,tokens", [(1, (33, 64, 65)), (48, (64, 65)), (512, (17, 24, 25)), (1100, (11, 12)), (6200, (1, 2))])
+def test_f32_limits(qgl, rows, tokens):
+    check(0, rows, 256, tokens)
+
+
+def test_f32_few_rows_stay_on_the_vector_chains(qgl):
+    """48 x 6144 takes no longer at 33 tokens than at 32 (the matrix-core tiles take 1.8 times as long)."""
+    assert graph_us(0, 48, 6144, 33) < 1.3 * graph_us(0, 48, 6144, 32)
