@@ -109,7 +109,7 @@ __global__ __launch_bounds__(64) void mm_exact_kernel(float *__restrict__ out, c
 }
 
 // qg_matmul for Q4_K and IQ4_NL rows with cols a multiple of 256 at up to 4
-// tokens: the arithmetic of mm_exact_kernel (the same weight value per
+// tokens (8 for small matrices): the arithmetic of mm_exact_kernel (the same weight value per
 // element, lane j's chain over k = j (mod 32) in ascending k, the same tree).
 // A block holds 8 rows, one per 32-lane half.  Per chunk of KC columns: the
 // rows' weight bytes and the tokens' x rows arrive by direct global->shared
@@ -119,6 +119,7 @@ __global__ __launch_bounds__(64) void mm_exact_kernel(float *__restrict__ out, c
 template <int TT> struct MmTile;
 template <> struct MmTile<1> { static constexpr int KC = 4096; };
 template <> struct MmTile<4> { static constexpr int KC = 2048; };
+template <> struct MmTile<8> { static constexpr int KC = 512; };
 
 template <int TYPE, int TT, int KCO = 0>
 __global__ __launch_bounds__(256) void mm_tile_kernel(float *__restrict__ out, const uint8_t *__restrict__ w, int rows,
@@ -269,10 +270,17 @@ void launch_mm_exact(float *out, const uint8_t *w, int type, int rows, int cols,
     if constexpr (TYPE == QT_Q4_K || TYPE == QT_IQ4_NL) {
         if (aligned && cols % 256 == 0) {
             // the vector chains up to 4 tokens (Q4_K 10240 x 2560: 15.2 us at 4
-            // tokens against 20.9), the matrix cores from 5 on (8 tokens: 26.3
-            // against 21.2 us, 17: 40.4 against 27.4, 1000: 1392 against 613)
+            // tokens against 20.9), the matrix cores from 9 on (17 tokens: 40.4
+            // against 27.4, 1000: 1392 against 613).  At 5..8 tokens a small
+            // matrix has too few tiles: two 4-token blocks (Q4_K, us, these / tiles:
+            // 512 x 512 4.2 / 5.3, 2048 x 2560 10.1 / 11.4, 6144 x 1024 9.0 / 9.3; 6144 x
+            // 2048 15.3 / 13.7) or, for many short rows, 8-token blocks (6144 x 512
+            // 6.1 / 6.9, 16384 x 256 7.3 / 8.2; 768 columns 7.7 / 8.2, 10240 rows 11.2 / 10.2).
             if (nt == 1) launch_mm_tile<TYPE, 1>(out, w, rows, cols, x, nt, stride, s);
             else if (nt <= 4) launch_mm_tile<TYPE, 4>(out, w, rows, cols, x, nt, stride, s);
+            else if (nt <= 8 && cols <= 512 && rows > 2048)
+                mm_tile_kernel<TYPE, 8><<<(rows + 7) / 8, 256, 0, s>>>(out, w, rows, cols, x, nt, stride);
+            else if (nt <= 8 && (long)rows * cols <= 6144L * 1024) launch_mm_tile<TYPE, 4>(out, w, rows, cols, x, nt, stride, s);
             else launch_xm<TYPE>(out, w, rows, cols, x, nt, stride, s);
             return;
         }

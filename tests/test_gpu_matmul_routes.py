@@ -62,3 +62,16 @@ def test_f32_limits(qgl, rows, tokens):
 def test_f32_few_rows_stay_on_the_vector_chains(qgl):
     """48 x 6144 takes no longer at 33 tokens than at 32 (the matrix-core tiles take 1.8 times as long)."""
     assert graph_us(0, 48, 6144, 33) < 1.3 * graph_us(0, 48, 6144, 32)
+
+
+@pytest.mark.parametrize("typ", [12, 20])
+@pytest.mark.parametrize("rows,cols", [(7, 256), (2048, 768), (2057, 512), (2057, 768), (2457, 2560), (2458, 2560)])
+def test_quantised_5_to_8_tokens(qgl, typ, rows, cols):
+    check(typ, rows, cols, (5, 7, 8, 9))
+
+
+@pytest.mark.parametrize("typ,rows,cols", [(12, 512, 512), (12, 6144, 256), (20, 6144, 256)])
+def test_quantised_5_tokens_against_the_tiles(qgl, typ, rows, cols):
+    """5 tokens of a small matrix take less time than 9, which the matrix-core tiles serve (their time is the same
+    at 5..16 tokens: 5.3 us against 4.1, 5.9 against 4.8, 5.6 against 5.1)."""
+    assert graph_us(typ, rows, cols, 5) < 0.97 * graph_us(typ, rows, cols, 9)
