@@ -328,18 +328,21 @@ __global__ __launch_bounds__(512, OCC) void xm_kernel(XmArgs A) {
     }
 }
 
-// Tile choice between 16 rows x 16 tokens (3 workgroups per CU) and 32 x 32 (2
-// per CU, half the operand reads and decoding per product): whether the wide
-// tile is the faster.  Estimated cost of a launch, in tenths of one full round
-// of the small tile, fitted to 2560-column timings: wide rounds of 512
-// workgroups take twice as long (31 against 16 us), 1.4 times while every CU
-// has one (22 us); so the wide tile is taken where it saves rounds (Q4_K 6144
-// x 2560, 300 tokens: 126 against 163 us) and the small one where the wide
-// leaves CUs idle (IQ4_NL 2560 x 6144, 33 tokens: 34 against 55 us).
-static inline bool xm_wide(int rows, int nt) {
-    const long b16 = (long)((rows + 15) / 16) * ((nt + 15) / 16), b32 = (long)((rows + 31) / 32) * ((nt + 31) / 32);
-    return (b32 <= 256 ? 14 : 20 * ((b32 + 511) / 512)) <= 10 * ((b16 + 767) / 768);
+// Estimated cost of a launch of tiles of `tr` rows x `tt` tokens, in tenths of
+// one full round of the small tile (16 x 16, 3 workgroups per CU), fitted to
+// 2560-column timings: the small tile in rounds of 768 workgroups; the wide
+// ones (32 x 32, 16 x 64; 2 per CU, half the operand reads and decoding per product)
+// in rounds of 512 that take twice as long (31 against 16 us), 1.4 times while
+// every CU has one (22 us).
+static inline long xm_cost(int rows, int nt, int tr, int tt) {
+    const long b = (long)((rows + tr - 1) / tr) * ((nt + tt - 1) / tt);
+    if (tr * tt == 256) return 10 * ((b + 767) / 768);
+    return b <= 256 ? 14 : 20 * ((b + 511) / 512);
 }
+// Whether 32 x 32 tiles are faster than 16 x 16: where they save rounds (Q4_K
+// 6144 x 2560, 300 tokens: 126 against 163 us), and not where they leave CUs idle
+// (IQ4_NL 2560 x 6144, 33 tokens: 34 against 55 us).
+static inline bool xm_wide(int rows, int nt) { return xm_cost(rows, nt, 32, 32) <= xm_cost(rows, nt, 16, 16); }
 
 template <int TYPE, int N16, int N4, int RR, int CH, int XR, int RS, int OCC>
 void xm_run(XmArgs A, hipStream_t s) {

@@ -243,14 +243,16 @@ void launch_mm_tile(float *out, const uint8_t *w, int rows, int cols, const floa
 template <int TYPE>
 void launch_xm(float *out, const uint8_t *w, int rows, int cols, const float *x, int nt, size_t stride, hipStream_t s) {
     const XmArgs A{out, rows, w, stride, rows, cols, x, nt, nullptr, 0, 0};
-    if constexpr (TYPE != QT_Q8_0) {
-        if (nt > 20 && xm_wide(rows, nt)) {
-            // IQ4_NL weights take more instructions to decode: 64 tokens share
-            // each instead of 32 (z 6144 x 2560, 2048 tokens: 802 -> 759 us)
-            if constexpr (TYPE == QT_IQ4_NL) xm_run<TYPE, 4, 0, 1, 1, 2, 4, 4>(A, s);
-            else xm_run<TYPE, 2, 0, 2, 1, 2, 4, 4>(A, s);
-            return;
-        }
+    if constexpr (TYPE == QT_IQ4_NL) {
+        // Its weights take more instructions to decode: in 16 x 64 tiles 64
+        // tokens share each, instead of 32 (6144 x 2560, 2048 tokens: 802 -> 759
+        // us); 32 x 32 where those would be mostly padding (10240 x 2560, 24
+        // tokens: 53 -> 37 us, 70: 94 -> 70; 6144 x 2560, 130: 93 -> 71).
+        const long c64 = xm_cost(rows, nt, 16, 64), c32 = xm_cost(rows, nt, 32, 32), c16 = xm_cost(rows, nt, 16, 16);
+        if (nt > 20 && c64 <= c32 && c64 <= c16) { xm_run<TYPE, 4, 0, 1, 1, 2, 4, 4>(A, s); return; }
+        if (nt > 20 && c32 <= c16) { xm_run<TYPE, 2, 0, 2, 1, 2, 4, 4>(A, s); return; }
+    } else if constexpr (TYPE != QT_Q8_0) {
+        if (nt > 20 && xm_wide(rows, nt)) { xm_run<TYPE, 2, 0, 2, 1, 2, 4, 4>(A, s); return; }
     }
     if constexpr (TYPE == QT_F32) {  // rows may be an odd number of chunks; 20-token tiles lose (512 x 2048: 10.0 against 7.6 us)
         xm_run<TYPE, 1, 0, 1, 1, 3, 4, 4>(A, s);

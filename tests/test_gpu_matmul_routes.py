@@ -75,3 +75,15 @@ def test_quantised_5_tokens_against_the_tiles(qgl, typ, rows, cols):
     """5 tokens of a small matrix take less time than 9, which the matrix-core tiles serve (their time is the same
     at 5..16 tokens: 5.3 us against 4.1, 5.9 against 4.8, 5.6 against 5.1)."""
     assert graph_us(typ, rows, cols, 5) < 0.97 * graph_us(typ, rows, cols, 9)
+
+
+@pytest.mark.parametrize("rows,tokens", [(512, (21, 65)), (2560, (70,)), (6144, (33, 130)), (10240, (21, 32, 33, 65))])
+def test_iq4nl_tile_choices(qgl, rows, tokens):
+    check(20, rows, 256, tokens)
+
+
+@pytest.mark.parametrize("rows,nt", [(10240, 24), (10240, 70), (6144, 130)])
+def test_iq4nl_tiles_as_q4k(qgl, rows, nt):
+    """IQ4_NL, whose weights take somewhat more to decode, stays near Q4_K of the same sizes (at most 13 % behind over
+    17..1024 tokens where both take the same tile) where 64-token tiles would be mostly padding (1.45 to 1.6 times)."""
+    assert graph_us(20, rows, 2560, nt) < 1.25 * graph_us(12, rows, 2560, nt)
