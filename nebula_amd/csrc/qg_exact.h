@@ -344,10 +344,25 @@ static inline long xm_cost(int rows, int nt, int tr, int tt) {
 // (IQ4_NL 2560 x 6144, 33 tokens: 34 against 55 us).
 static inline bool xm_wide(int rows, int nt) { return xm_cost(rows, nt, 32, 32) <= xm_cost(rows, nt, 16, 16); }
 
+// Token tiles per launch (at least 1) of a matrix with nrt row tiles.
+static inline int xm_slice(int nrt) {
+    constexpr int TILES = (1 << 23) - 1;
+    const int n = TILES / nrt;
+    return n < 1 ? 1 : n > QG_MAX_TOKENS ? QG_MAX_TOKENS : n;
+}
+// A launch holds fewer than 2^32 threads, 2^23 tiles: more (Q8_0 outputs of 2^31 and
+// more elements) go out in slices of whole token tiles.  Rows alone stay below
+// that (a matrix of 2^27 rows is past what the vector chains' launch takes, too).
 template <int TYPE, int N16, int N4, int RR, int CH, int XR, int RS, int OCC>
 void xm_run(XmArgs A, hipStream_t s) {
     using S = XmShape<TYPE, N16, N4, RR, CH, XR, RS>;
-    A.ntt = (A.nt + S::TOK - 1) / S::TOK;
     A.nrt = (A.rows + S::ROWS - 1) / S::ROWS;
-    xm_kernel<TYPE, N16, N4, RR, CH, XR, RS, OCC><<<A.ntt * A.nrt, 512, S::LDS, s>>>(A);
+    const int nt = A.nt, most = xm_slice(A.nrt) * S::TOK;
+    for (int t = 0; t < nt; t += most) {
+        A.nt = nt - t < most ? nt - t : most;
+        A.ntt = (A.nt + S::TOK - 1) / S::TOK;
+        xm_kernel<TYPE, N16, N4, RR, CH, XR, RS, OCC><<<A.ntt * A.nrt, 512, S::LDS, s>>>(A);
+        A.out += (size_t)most * A.ldo;
+        A.x += (size_t)most * A.cols;
+    }
 }

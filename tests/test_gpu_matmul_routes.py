@@ -87,3 +87,30 @@ def test_iq4nl_tiles_as_q4k(qgl, rows, nt):
     """IQ4_NL, whose weights take somewhat more to decode, stays near Q4_K of the same sizes (at most 13 % behind over
     17..1024 tokens where both take the same tile) where 64-token tiles would be mostly padding (1.45 to 1.6 times)."""
     assert graph_us(20, rows, 2560, nt) < 1.25 * graph_us(12, rows, 2560, nt)
+
+
+def test_output_past_one_launch(qgl):
+    """Q8_0, 1048592 rows x 2064 tokens: 65537 row tiles x 129 token tiles are more workgroups than one launch holds
+    (2^23 - 1 of 512 threads); the output has 2.2e9 elements.  Sampled rows of the tokens around the cut (127 token
+    tiles, 2032 tokens) and at both ends, bit for bit."""
+    rows, cols, nt = 65537 * 16, 256, 2064
+    rng = np.random.default_rng(8)
+    w = np.ascontiguousarray(legal_blocks(rng, 8, 4096, cols))
+    w = np.ascontiguousarray(np.resize(w, (rows, w.shape[1])))   # the 4096 rows, repeated
+    w[-16:] = legal_blocks(rng, 8, 16, cols)
+    x = rng.normal(0, .5, (nt, cols)).astype(np.float32)
+    dw, dx = Device(w), Device(x)
+    out = qg.lib().qg_alloc(rows * nt * 4)
+    assert out
+    try:
+        print(f"matmul past one launch {rows}x{cols} nt={nt}", flush=True, file=sys.stderr)
+        call("matmul", out, dw.p, 8, rows, cols, dx.p, nt)
+        call("sync")
+        pick = np.r_[0:40, 4080:4112, rows // 2:rows // 2 + 16, rows - 32:rows]
+        for t in (0, 1000, 2031, 2032, 2047, 2048, nt - 1):
+            got = np.empty(rows, np.float32)
+            call("read", got.ctypes.data, out + t * rows * 4, got.nbytes)
+            want = O.matmul(np.ascontiguousarray(w[pick]), 8, len(pick), cols, x[t:t + 1])[0]
+            np.testing.assert_array_equal(got[pick].view('u4'), want.view('u4'), err_msg=f"token {t}")
+    finally:
+        qg.lib().qg_free(out)
