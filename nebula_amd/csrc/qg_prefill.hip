@@ -239,9 +239,14 @@ QG_DEV int scan512(int v, int *s_tmp) {
     return v + base;
 }
 
-// Rows per tile unit (TM, in tiles of 8 rows) of the short-list kernels that a
-// batch's gate/up and down may take, 0 where nothing is left to decide.
-struct SpForms { int gu, dn; };
+// Rows per run (TM, in tiles of 8 rows) of the short-list kernels that a batch's
+// gate/up and down may take, 0 where nothing is left to decide; 128-row blocks of
+// F and workgroups of a gate/up on the 64-row tiles.
+struct SpForms { int gu, dn, blocks, cus; };
+
+// The 64-row tiles are taken below this ratio of the two prices (measured, see
+// sp_forms).
+constexpr float SP_GU_RATIO = 1.95f, SP_DN_RATIO = 1.67f;
 
 // Price of a list of n rows on a short-list kernel with runs of 8 TM rows
 // (qg_sparse.h), in the same unit for any TM.
@@ -330,11 +335,13 @@ QG_DEV void tile_table(TileTable *tt, int n, int shared_rows, SpForms sp, int *s
         }
         tt->bounds[3] = all;
         tt->mbounds[3] = mall;
-        // 64-row tiles where their price (7 + 3 M per tile of M 16-row steps, as
-        // balanced_items) is below 5/3 of the short-list kernels'
-        const int tiles = 3 * (7 * all + 3 * mall);
-        tt->tiles_gu = sp.gu && tiles < 5 * ((price >> 16) + sp_price(shared_rows, sp.gu));
-        tt->tiles_dn = sp.dn && tiles < 5 * ((price & 0xffff) + sp_price(shared_rows, sp.dn));
+        // the 64-row tiles' price is 7 + 3 M per tile of M 16-row steps, as in
+        // balanced_items; gate/up items are so long that the last round of
+        // workgroups counts halfway as a whole one
+        const int tiles = 7 * all + 3 * mall, items = all * sp.blocks, full = (items + sp.cus - 1) / sp.cus * sp.cus;
+        const float gu = (float)((price >> 16) + sp_price(shared_rows, sp.gu));
+        tt->tiles_gu = sp.gu && (float)tiles * (float)(items + full) < 2.0f * SP_GU_RATIO * gu * (float)items;
+        tt->tiles_dn = sp.dn && (float)tiles < SP_DN_RATIO * (float)((price & 0xffff) + sp_price(shared_rows, sp.dn));
     }
 }
 
@@ -1459,12 +1466,12 @@ __global__ __launch_bounds__(512, 1) void pf_down_pick_kernel(SpDnArgs S, DnArgs
 // Second, below those sizes, by the rows of the lists, which only the device
 // knows: tokens of one context share their experts, and a list of n rows is
 // converted n / 24 or n / 16 times (IQ4_NL down: n / 8) against n / 64.
-// tile_table compares the two forms' prices over the batch's lists.  The factor
-// 5/3 comes from times of both over 18..1280 tokens of uniform, Zipf, loosely
-// and closely related tokens, every shape above (336 points): the rule's choice is
-// on average 0.4 % and at most 12 % behind the better one, always the short-list
-// kernel 14 % (2048/512 IQ4_NL, 448 closely related tokens: gate/up 82 / 73 us, down
-// 91 / 40; 2560/640: 146 / 90, 133 / 62).  Where both forms have the same
+// tile_table compares the two forms' prices over the batch's lists.  The ratios
+// come from times of both over 65..1400 tokens of uniform, Zipf, loosely and
+// closely related tokens, thirteen shapes: gate/up (154 batches) is on average 0.3 %
+// and at most 12 % behind the better form, always the short-list kernel 14 %; down
+// (100) 0.7 %, always the short-list kernel 24 % (2048/512 IQ4_NL, 448 closely related
+// tokens: gate/up 82 / 73 us, down 91 / 40; 2560/640: 146 / 90, 133 / 62).  Where both forms have the same
 // workgroups they are one kernel; gate/up at D = 2560 and 1024, whose short-list
 // kernels have 640 and 256 threads, takes two launches of which one is idle (2.5
 // us), from the batch on at which the tiles can be ahead by more than that.
@@ -1475,7 +1482,7 @@ __global__ __launch_bounds__(512, 1) void pf_down_pick_kernel(SpDnArgs S, DnArgs
 // take the FULL forms.
 constexpr int sp_down_tm(int fmt, int nb) { return fmt == QT_IQ4_NL && nb >= 16 ? 1 : 2; }
 SpForms sp_forms(int D, int F, int down_fmt, int nt) {
-    SpForms f{0, 0};
+    SpForms f{0, 0, F / GU_FB, qg_cu_count()};
     if (D == 2048 && nt <= 1280) f.gu = 3;
     if ((D == 2560 && nt <= 640) || (D == 1024 && nt <= 896)) f.gu = 2;
     const int most = down_fmt == QT_Q4_K ? (F == 256 ? 768 : F == 512 ? 1280 : 0) : (F == 256 ? 640 : F == 512 || F == 640 ? 448 : 0);
@@ -1484,7 +1491,7 @@ SpForms sp_forms(int D, int F, int down_fmt, int nt) {
 }
 // The forms of which the device chooses by the lists.
 SpForms sp_ask(const SpForms &f, int D, int nt) {
-    return SpForms{nt > (D >= 2048 ? 128 : 384) ? f.gu : 0, nt > 64 ? f.dn : 0};
+    return SpForms{nt > (D >= 2048 ? 128 : 384) ? f.gu : 0, nt > 64 ? f.dn : 0, f.blocks, f.cus};
 }
 // gate/up where sp_forms(...).gu is not 0
 int pf_gateup_sp(const SpGuArgs &A, const GuArgs &T, int cus, hipStream_t s) {
@@ -1790,7 +1797,7 @@ int qg_prefill_dispatch(int *offsets, int *row_token, int *row_slot, int *status
     pf_count_kernel<<<nch, 512, 0, s>>>(counts, bad, ids, nullptr, nt);
     int rc = hipGetLastError();
     if (rc) return rc;
-    pf_scan_kernel<<<1, 512, 0, s>>>(counts, nch, offsets, nullptr, 0, SpForms{0, 0}, bad, status);
+    pf_scan_kernel<<<1, 512, 0, s>>>(counts, nch, offsets, nullptr, 0, SpForms{}, bad, status);
     if ((rc = hipGetLastError())) return rc;
     pf_fill_kernel<<<nch, 512, 0, s>>>(row_token, row_slot, counts, ids, nullptr, nt, nullptr, nullptr);
     return hipGetLastError();
