@@ -35,12 +35,6 @@ QG_DEV int plane_pos(int fmt, int k) {
     return fmt == QT_IQ4_NL ? (k & ~31) | pos_iq4(k & 31) : (k & ~255) | pos_q4k(k & 255);
 }
 
-// The 8 fp16 values s*q of one fragment of a Q4_K qs chunk (c = 16 bytes):
-// f bit 1 = high nibbles, f bit 0 = bytes 8..15.
-QG_DEV qg_half8 q4k_chunk_frag(uint4 c, int f, _Float16 s) {
-    return q4_frag((f & 1) ? make_uint2(c.z, c.w) : make_uint2(c.x, c.y), f >> 1, s);
-}
-
 // 4 IQ4_NL qs bytes -> 8 table values in fp16, slots 0..3 / 4..7 = low /
 // high nibbles of bytes 0..3 (pos_iq4's order).  The table bytes (value +
 // 128) are permuted in pairs under the exponent byte 0x64 (1024 + value +

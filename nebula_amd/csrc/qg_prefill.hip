@@ -1,6 +1,7 @@
 // Routed-MoE layer for prefill batches (18..8192 tokens): the path of
-// qg_moe_forward / qg_moe_forward_residual above the decode sizes, for Q4_K
-// gate/up and Q4_K or IQ4_NL down.  It replaces the per-expert loop of
+// qg_moe_forward / qg_moe_forward_residual above the decode sizes (and of decode
+// batches at D = 1024, see qg_prefill_small_ok), for Q4_K gate/up and Q4_K or
+// IQ4_NL down.  It replaces the per-expert loop of
 // qwen.c:680-700 (qg_moe_map, then qg_matmul x3 and qg_moe_scatter per expert,
 // or qc_moe of cpu.c:235-261 on the CPU handoff) with grouped GEMMs over
 // per-expert row lists built on the device.
@@ -664,8 +665,8 @@ constexpr int IQ_STAGE = PT * 2 * IQ_KC * 2;        // [64 rows][2 planes][128] 
 constexpr int PF_IQ_LDS = 2 * IQ_STAGE + PF_WAVES * 3 * IQ_SLOT;
 static_assert(32 * IQ_PIECES <= IQ_COPIES * 64, "the copies cover the slot");
 
-// Activation stage of one 128-element K chunk: [row][plane][16 chunks of 16
-// bytes], chunk position c ^ (row & 15); one copy covers two rows.
+// 16-byte chunk c of row r, plane p of a 128-element activation stage:
+// [row][plane][16 chunks], chunk c at position c ^ (row & 15).
 QG_DEV qg_half8 stage_frag128(const uint8_t *st, int r, int p, int c) {
     return ld_frag((const _Float16 *)(st + (r * 2 + p) * 256 + 16 * (c ^ (r & 15))));
 }
@@ -907,11 +908,9 @@ constexpr int GQ_SUMS = PT * 2 * 16;                 // [64 rows][2 planes][8 gr
 constexpr int PF_GQ_LDS = 2 * IQ_STAGE + 2 * GQ_SUMS + PF_WAVES * 3 * GQ_SLOT;
 static_assert(32 * GQ_PIECES <= GQ_COPIES * 64, "the copies cover the slot");
 
-// The int8 variant's stage of one 128-element K chunk: [row][plane][8 chunks
-// of 16 bytes] (natural K order), chunk position c ^ (row & 7); one copy
-// covers four rows.
-// 8 int8 activations of row r, plane p: elements 8 kq .. 8 kq + 7 of group f
-// of the chunk.
+// 8 int8 activations of row r, plane p, elements 8 kq .. 8 kq + 7 of group f,
+// of the int8 variant's 128-element stage: [row][plane][8 chunks of 16 bytes] in
+// natural K order, chunk c at position c ^ (row & 7).
 QG_DEV long stage_frag128_i8(const uint8_t *st, int r, int p, int f, int kq) {
     return *(const long *)(st + r * 256 + p * 128 + 16 * ((2 * f + (kq >> 1)) ^ (r & 7)) + 8 * (kq & 1));
 }
