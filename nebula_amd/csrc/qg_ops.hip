@@ -251,7 +251,7 @@ void launch_xm(float *out, const uint8_t *w, int rows, int cols, const float *x,
         const long c64 = xm_cost(rows, nt, 16, 64), c32 = xm_cost(rows, nt, 32, 32), c16 = xm_cost(rows, nt, 16, 16);
         if (nt > 20 && c64 <= c32 && c64 <= c16) { xm_run<TYPE, 4, 0, 1, 1, 2, 4, 4>(A, s); return; }
         if (nt > 20 && c32 <= c16) { xm_run<TYPE, 2, 0, 2, 1, 2, 4, 4>(A, s); return; }
-    } else if constexpr (TYPE != QT_Q8_0) {
+    } else if constexpr (TYPE != QT_Q8_0) {  // (a wave's share of 32 Q8_0 rows is 68 pieces, more than one copy instruction's)
         if (nt > 20 && xm_wide(rows, nt)) { xm_run<TYPE, 2, 0, 2, 1, 2, 4, 4>(A, s); return; }
     }
     if constexpr (TYPE == QT_F32) {  // rows may be an odd number of chunks; 20-token tiles lose (512 x 2048: 10.0 against 7.6 us)

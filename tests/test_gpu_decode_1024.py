@@ -144,3 +144,40 @@ def test_decode_phase_events(qgl, nt):
         qg.call("moe_phase_events", None, 0)
         for e in events:
             qgl.qg_event_destroy(e)
+
+
+@pytest.mark.parametrize("nt", [1, 17])
+def test_decode_in_a_replayed_graph(qgl, nt):
+    """Direct and residual form in one graph, replayed on other inputs, against the eager calls' bits."""
+    L, _ = make("512-q4k")
+    fw = synth.Forward(1024, 512, nt)
+    h, xn, out = (qg.Device(shape=(nt, 1024), dtype=np.float32) for _ in range(3))
+
+    def calls():
+        fw.run(L, nt)
+        qg.call("moe_forward_residual", h.p, fw.ids.p, fw.w.p, fw.flags.p, None, xn.p, out.p, nt, qg.C.byref(L.desc), fw.ws.p, fw.ws_bytes)
+
+    def results():
+        qg.call("sync")
+        return [d.get()[:nt].view('u4') for d in (fw.out, h, xn, out)]
+
+    xs = [synth.inputs(650 + k, nt, 1024, correlated=k == 1) for k in range(3)]
+    want = []
+    for x in xs:
+        fw.x.set(x)
+        h.set(3 * x)
+        calls()
+        want.append(results())
+    graph = qg.C.c_void_p()
+    qg.call("graph_begin", qg.C.byref(graph))
+    calls()
+    qg.call("graph_end", graph)
+    try:
+        for k in (0, 1, 2, 0):
+            fw.x.set(xs[k])
+            h.set(3 * xs[k])
+            qg.call("graph_launch", graph)
+            for a, b in zip(results(), want[k]):
+                np.testing.assert_array_equal(a, b, err_msg=f"nt={nt} input {k}")
+    finally:
+        qg.lib().qg_graph_destroy(graph)

@@ -76,3 +76,26 @@ def test_one_context_costs_no_more_below_the_limit(case, which):
     print(f"limit {name} {which} nt={nt}: {below:.1f} us, one token more {above:.1f}", flush=True, file=sys.stderr)
     # the short-list kernels would take 1.2 to 2.2 times as long; an idle launch is up to 4 us
     assert below < 1.12 * above + 4
+
+
+def test_choice_in_a_replayed_graph(case):
+    """The choice is made at each replay: a graph captured on independent tokens and replayed on tokens of one context, and
+    back, gives the eager calls' bits."""
+    name, L, _ = case
+    nt = LIMITS[name][3]
+    xs = [synth.inputs(740, nt, L.spec.width), S.one_context(741, nt, L.spec.width)]
+    want = [P.forward(L, x).out.get()[:nt] for x in xs]
+    fw, graph = synth.Forward(L.spec.width, L.spec.ff, nt), qg.C.c_void_p()
+    fw.x.set(xs[0])
+    fw.run(L, nt)
+    qg.call("graph_begin", qg.C.byref(graph))
+    fw.run(L, nt)
+    qg.call("graph_end", graph)
+    try:
+        for k in (0, 1, 1, 0):
+            fw.x.set(xs[k])
+            qg.call("graph_launch", graph)
+            qg.call("sync")
+            np.testing.assert_array_equal(fw.out.get()[:nt].view('u4'), want[k].view('u4'), err_msg=f"{name} input {k}")
+    finally:
+        qg.lib().qg_graph_destroy(graph)
